@@ -75,10 +75,10 @@ def bytes_per_chunk(kernel, c, d=D):
         "fwd_scan": e + 2 * tile + s + sq + tile,
         # q, k, rk, gcum, h^T, v_new^T -> o
         "fwd_out": 2 * e + 2 * s + sq + tile + e,
-        # q, k, rk, dO, gcum, beta, T -> dv_local^T, X^T, kdec Kn perm32, -W^T
-        "bwd_local": 3 * e + 3 * s + tm + tile + sq + e + tile,
-        # kdec Kn perm32, gcum, dv_local^T, X^T, -W^T -> dh, dv_new (both value-slice-major)
-        "bwd_scan": e + s + tile + sq + tile + sq + tile,
+        # q, k, rk, dO, gcum, beta, T -> dv_local^T, X^T, kdec Kn and -W^T fragments
+        "bwd_local": 3 * e + 3 * s + tm + tile + sq + 2 * tile,
+        # kdec Kn and -W^T fragments, gcum, dv_local^T, X^T -> dh, dv_new (both value-slice-major)
+        "bwd_scan": 2 * tile + s + tile + sq + sq + tile,
         # q, k, rk, gcum, h^T, v_new^T, dO, dh, dv_new, v, beta, T -> dq, dk, dv, dg, dbeta
         "bwd_dkw": 2 * e + 2 * s + sq + tile + e + sq + tile + e + s + tm + 3 * e + 2 * s,
     }[kernel]

@@ -134,18 +134,16 @@ __global__ __launch_bounds__(256, 3) void bwd_local_kernel(
   }
   __syncthreads();
 
-  // perm32 copy of kdec_t Kn_t (kdec_t = exp(G_last - G_t), the decay the
-  // reverse scan applies to Kn dS) from the tile: 16-byte piece p of column
-  // block j holds logical 32 j + 4 p .. + 3 and 32 j + 16 + 4 p .. + 3
+  // kdec_t Kn_t (kdec_t = exp(G_last - G_t), the decay the reverse scan applies to Kn dS)
+  // in the order the scan reads it: fragment (t / 16, k / 32), and in it 16-byte granule
+  // 16 g + r holding row t = 16 (t / 16) + r, k = 32 (k / 32) + 8 g ..
   {
-    const int t = tid >> 2, p = tid & 3;
-    if (t < ci.len) {
-      const float kd = __expf(Gs[ci.len - 1] - Gs[t]);
-      E* kp = knP + ((size_t)(ci.start + t) * H + h) * D + 8 * p;
+    E* kp = knP + cb * (CH * D) + 8 * tid;
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
-        st8(kp + 32 * j, cat(to4<E>(cvtf4(ld4(Ks + t * LDK + 32 * j + 4 * p)) * kd),
-                             to4<E>(cvtf4(ld4(Ks + t * LDK + 32 * j + 16 + 4 * p)) * kd)));
+    for (int i = 0; i < 4; ++i) {
+      const int t = 16 * i + r;
+      const float kd = __expf(Gs[ci.len - 1] - Gs[t]);
+      st8(kp + 2048 * i, to8<E>(cvtf8(ld8(Ks + t * LDK + 32 * wave + 8 * q4)) * kd));
     }
   }
 
@@ -160,10 +158,14 @@ __global__ __launch_bounds__(256, 3) void bwd_local_kernel(
       fbg[kb][e] = Bs[s] * fg[kb][e];
     }
 
-  // -W^T [k][perm32(t)] with W = T (beta gam K): t-tile = wave, k-tiles n; beta gam K
-  // is read transposed from the K rows and scaled per event s on the way
+  // -W^T with W = T (beta gam K): t-tile = wave, k-tiles n; beta gam K is read transposed
+  // from the K rows and scaled per event s on the way.  Stored in the order the reverse
+  // scan reads it: fragment (k / 32, (k / 4) % 2, t / 32), and in it granule 16 g + i
+  // holding row k = .. + 8 (i / 4) + i % 4 at the four-runs g of both halves of the 32
+  // events (perm32)
   {
-    E* wt = WT + cb * (D * CH);
+    E* wt = WT + cb * (D * CH) + (64 * (2 * ((r >> 2) & 1) + (wave >> 1)) + 16 * q4 + 4 * (r >> 3) + (r & 3)) * 8 +
+            4 * (wave & 1);
 #pragma unroll
     for (int n = 0; n < 8; ++n) {
       f32x4 aw = zero4();
@@ -171,7 +173,7 @@ __global__ __launch_bounds__(256, 3) void bwd_local_kernel(
       for (int kb = 0; kb < 2; ++kb)
         if (kb == 0 || wave >= 2)  // T[t][s] = 0 for s > t
           aw = mfma(at[kb], to8<E>(cvtf8(ld8_tr(Ks, LDK, 32 * kb, 16 * n)) * fbg[kb]), aw);
-      st4(wt + (16 * n + r) * CH + perm32(16 * wave + 4 * q4), -aw);
+      st4(wt + (n >> 1) * 2048 + (n & 1) * 64, -aw);
     }
   }
 
@@ -258,132 +260,26 @@ __global__ __launch_bounds__(256, 3) void bwd_local_kernel(
 }
 
 // ---------------------------------------------------------------------------
-// bwd_state: one wave per (head, 16-wide value slice, document), chunks in reverse
+// bwd_scan: the reverse scan, four waves per (head, 16-wide value slice, document)
 // ---------------------------------------------------------------------------
-// Reverse scan, organised like fwd_scan_kernel: one consumer wave per (head,
-// 16-wide value slice), two loader waves copying each chunk's operands
-// global -> LDS asynchronously into a 4-stage ring, BS_DEPTH chunks ahead, each
-// loader issuing its own part of every chunk (part 0: kdec Kn, G_last, X^T;
-// part 1: -W^T, dv_local^T).  The consumer's output tiles (dS^T, dVn^T) go into the
-// stage region it has read (-W^T) and are stored by loader 1, which refills
-// that region right after.  Tiles use the same XOR swizzles as the forward
-// scan:
-//   Kn  [64 rows t][16 cols]   col ^ (t & 15)      W^T [128 rows k][8 cols]  col ^ ((k >> 1) & 7)
-//   X^T [16 rows v][16 cols]   col ^ (v & 15)      dv_local^T [16 rows v][8 cols]  col ^ ((v >> 1) & 7)
-constexpr int BS_THREADS = 64 * 3;
-constexpr int BS_DEPTH = 3;
-constexpr int BS_STAGES = 4;
-constexpr int BS_SROW = 136;
-constexpr int BS_VROW = 72;
-
-template <class E>
-struct __attribute__((aligned(16))) BwdStage {
-  E kn[64 * 128];   // Kn rows t
-  E wt[128 * 64];   // -W^T rows k
-  E dvl[16 * 64];   // dv_local^T rows of the slice
-  E xt[16 * 128];   // X^T rows of the slice
-  float glast;      // G of the chunk's last event
-  float pad[3];
-};
-
-template <class E>
-struct __attribute__((aligned(16))) BwdScratch {
-  E s[16 * BS_SROW];  // dS_{c+1}, [v][k]
-  E v[16 * BS_VROW];  // dVn, [v][t]
-};
-static_assert(sizeof(BwdScratch<bf16>) <= 128 * 64 * sizeof(bf16), "scratch must fit the -W^T region");
-template <class E>
-__device__ __forceinline__ BwdScratch<E>& bwd_scratch(BwdStage<E>& st) {
-  return *reinterpret_cast<BwdScratch<E>*>(st.wt);
-}
-
-// Issue part `part` of the asynchronous copies of chunk c into stage S (no
-// wait on memory here): part 0 kdec Kn, G_last and the X^T slice (21 copies),
-// part 1 (loader 1, which also stores the outputs) -W^T and the dv_local^T
-// slice (18 copies).
-constexpr int BWD_PART_COPIES[2] = {21, 18};
-template <class E>
-__device__ __forceinline__ void bwd_issue(BwdStage<E>& S, const int32_t* __restrict__ chunks, int c, int H, int h,
-                                          int v0, int lane, int part, const E* __restrict__ knP,
-                                          const float* __restrict__ gc, const E* __restrict__ dvlT,
-                                          const E* __restrict__ XT, const E* __restrict__ WT) {
-  const ChunkInfo ci = chunk_info(chunks, c);
-  const size_t cb = (size_t)c * H + h;
-  if (part == 0) {
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {  // rows past the tail re-read row len-1 and are zeroed by bwd_fix_tail
-      const int t = 4 * i + (lane >> 4), col = (lane & 15) ^ (t & 15);
-      const int tt = min(t, ci.len - 1);
-      dma16(knP + ((size_t)(ci.start + tt) * H + h) * D + 8 * col, S.kn + 512 * i);
-    }
-    if (lane == 0)  // one lane: a dword copy writes 4 bytes per active lane
-      __builtin_amdgcn_global_load_lds(gc + (size_t)(ci.start + ci.len - 1) * H + h, (lds_void_ptr)&S.glast, 4, 0,
-                                       0);
-    const E* xt = XT + cb * (D * D) + v0 * D;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int v = 4 * i + (lane >> 4), col = (lane & 15) ^ (v & 15);
-      dma16(xt + v * D + 8 * col, S.xt + 512 * i);
-    }
-  } else {
-    const E* wt = WT + cb * (D * CH);
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const int k = 8 * i + (lane >> 3), col = (lane & 7) ^ ((k >> 1) & 7);
-      dma16(wt + k * CH + 8 * col, S.wt + 512 * i);
-    }
-    const E* dvl = dvlT + cb * (D * CH) + v0 * CH;
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int v = 8 * i + (lane >> 3), col = (lane & 7) ^ ((v >> 1) & 7);
-      dma16(dvl + v * CH + 8 * col, S.dvl + 512 * i);
-    }
-  }
-}
-
-template <class E>
-__device__ __forceinline__ void bwd_fix_tail(BwdStage<E>& S, const int32_t* __restrict__ chunks, int c, int lane) {
-  const int len = chunk_info(chunks, c).len;
-  if (len < CH) {
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const int t = 4 * i + (lane >> 4);
-      if (t >= len) st8(S.kn + t * 128 + 8 * (lane & 15), zero8v<E>());
-    }
-  }
-}
-
-// global stores of one copy-out (4 of dS, 2 of dVn)
-constexpr int BWD_OUT_STORES = 6;
-
-// scratch of one step -> dS_{c+1} and dVn in value-slice-major blocks (the
-// slice's [k][16] and [t][16], read transposed from the [v][k] / [v][t] scratch).
-// Each store instruction writes 1 KB of contiguous lines, with the non-temporal
-// hint: the scan still has the earlier chunks' operands to read (bwd_local wrote
-// them first to last, so they are the oldest in the memory-side cache).  With
-// bwd_dkw beside the scan (SC1) the stores are device-scope: bwd_dkw reads them
-// while the scan runs.
-template <bool SC1, class E>
-__device__ __forceinline__ void bwd_copy_out(const BwdScratch<E>& sc, int c, int H, int h, int slice, int lane,
-                                             E* __restrict__ dhS, E* __restrict__ dVnS) {
-  const size_t cb = (size_t)c * H + h;
-  const int r = lane & 15, q4 = lane >> 4, half = 8 * (q4 & 1), row = 16 * (q4 >> 1) + r;
-  E* ds = dhS + cb * (D * D) + slice * (D * 16);
-  E* vs = dVnS + cb * (CH * D) + slice * (CH * 16);
-  if constexpr (SC1) {
-    const __amdgpu_buffer_rsrc_t dr = buf_rsrc(ds, D * 16 * 2), vr = buf_rsrc(vs, CH * 16 * 2);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) buf_st16_nt_sc1(dr, ((32 * i + row) * 16 + half) * 2, ld8_tr16(sc.s, BS_SROW, 32 * i));
-#pragma unroll
-    for (int i = 0; i < 2; ++i) buf_st16_nt_sc1(vr, ((32 * i + row) * 16 + half) * 2, ld8_tr16(sc.v, BS_VROW, 32 * i));
-  } else {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) st8_nt(ds + (32 * i + row) * 16 + half, ld8_tr16(sc.s, BS_SROW, 32 * i));
-#pragma unroll
-    for (int i = 0; i < 2; ++i) st8_nt(vs + (32 * i + row) * 16 + half, ld8_tr16(sc.v, BS_VROW, 32 * i));
-  }
-}
-
+// Organised as fwd_scan (gdn_fwd.hip): wave w holds rows 32 w .. of the slice's dS and
+// does a quarter of each contraction, dS and dVn pass through LDS with a barrier after
+// each.  bwd_local writes both matrices, kdec Kn and -W^T, in fragment order, so their
+// loads are 1 KB of contiguous operands; X^T and dv_local^T are read by quads and
+// exchanged between lanes; dS and dVn are read back from LDS transposed, as whole blocks
+// of the value-slice-major outputs.  The tiles' rows are k = 32 w + 8 (i / 4) + 4 m + i % 4,
+// so a lane's eight values of dS are consecutive in k: one 16-byte LDS write, and one
+// 16-byte piece of X^T.
+//
+// Measured (H = 16, one document of 144 chunks / 15 documents, 520 chunks): 116.6 -> 104.4
+// us, 331 -> 299 us; 36 chunks 32.4 -> 25.3; four heads, 144 chunks 113.6 -> 83.4; beside
+// bwd_dkw a step of 144 chunks went from 477 to 448 us, the scan (7 KB of LDS instead of
+// 152) now sharing its CUs with bwd_dkw workgroups.
+//
+// The outputs are stored with the non-temporal hint: the scan still has the earlier chunks'
+// operands to read (bwd_local wrote them first to last, so they are the oldest in the
+// memory-side cache).  With bwd_dkw beside it (SC1) the stores are device-scope, and the
+// waves run at a raised priority (four heads: a step 270 -> 266 us; no change at 16).
 // One slice's dS / dVn of chunk c are stored (their stores have completed): add to
 // the chunk's count, which bwd_dkw waits to see at 8, from one lane.
 __device__ __forceinline__ void bwd_publish(int* __restrict__ ready, int c, int H, int h, int lane) {
@@ -392,160 +288,166 @@ __device__ __forceinline__ void bwd_publish(int* __restrict__ ready, int c, int 
   asm volatile("" ::: "memory");
 }
 
-template <class E>
-__global__ __launch_bounds__(BS_THREADS) void bwd_scan_kernel(
-    const E* __restrict__ knP, const float* __restrict__ gc, const E* __restrict__ dvlT,
-    const E* __restrict__ XT, const E* __restrict__ WT, const int32_t* __restrict__ chunks,
-    const int32_t* __restrict__ doc_chunk, int H, E* __restrict__ dhS, E* __restrict__ dVnS,
-    int* __restrict__ ready, int* __restrict__ resident) {
-  // ready / resident: null, or the hand-off counts of a bwd_dkw running beside this
-  // scan (each workgroup adds one to resident when it starts, and one to a chunk's
-  // ready count once its outputs of that chunk are stored)
+// Vector memory operations of one full step of one wave: 8 operand fragments, X, dv_local,
+// two stores.  A step's chunk is announced BWD_ANNOUNCE steps later.
+constexpr int BWD_STEP_OPS = 12, BWD_ANNOUNCE = 3;
+
+template <class E, bool SC1>
+__global__ __launch_bounds__(SCAN_THREADS, 2) void bwd_scan_kernel(
+    // without __restrict__ where loads are requested ahead: the barriers then pin their place
+    const E* knP, const float* gc, const E* dvlT, const E* XT, const E* WT, const int32_t* chunks,
+    const int32_t* __restrict__ doc_chunk, int H, E* dhS, E* dVnS, int* ready, int* resident) {
+  // SC1: a bwd_dkw runs beside this scan (each workgroup adds one to resident when it
+  // starts, and one to a chunk's ready count once its outputs of that chunk are stored)
   typedef typename Vec<E>::x8 X8;
   typedef typename Vec<E>::x4 X4;
   const int h = blockIdx.x % H, slice = blockIdx.x / H, d = blockIdx.y;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r = lane & 15, q4 = lane >> 4;
   const int v0 = 16 * slice;
+  constexpr int OUT = CPOL_NT | (SC1 ? CPOL_SC1 : 0);
+  if constexpr (SC1) __builtin_amdgcn_s_setprio(3);
 
-  __shared__ BwdStage<E> stage[BS_STAGES];
+  __shared__ __attribute__((aligned(16))) E Sx[16 * SCAN_SROW];  // dS's operand copy, [v][k]
+  __shared__ __attribute__((aligned(16))) E Vx[16 * SCAN_VROW];  // dVn, [v][perm32(t)]
 
-  const int c_end = doc_chunk[d + 1], n = c_end - doc_chunk[d];
-  // step tau handles chunk c_end - 1 - tau (chunks in reverse)
-  if (wave == 0) {
-    if (resident && lane == 0) count_add(resident);
-    f32x4 dS[8];  // dS[m][i] = dState[k = 16m + 4q4 + i][v = v0 + r]
+  const int c_begin = __builtin_amdgcn_readfirstlane(doc_chunk[d]);
+  const int c_last = __builtin_amdgcn_readfirstlane(doc_chunk[d + 1]) - 1, n = c_last + 1 - c_begin;
+  if (SC1 && threadIdx.x == 0) count_add(resident);
+  if (n <= 0) return;
+  // step tau handles chunk c_last - tau
+  f32x4 dS[2];  // dS[m][i] = dState[k = 32 wave + 8 q4 + 4 m + i][v = v0 + r]
 #pragma unroll
-    for (int m = 0; m < 8; ++m) dS[m] = zero4();
-    int kofs[4], wofs[2], dofs[4], xofs[8];
+  for (int m = 0; m < 2; ++m) dS[m] = zero4();
+  ScanTable tab(chunks, gc, nullptr, c_last, -1, n, H, h, lane);
+  const size_t cb = (size_t)c_last * H + h;
+  const int64_t tile = (int64_t)H * D * CH * 2;  // bytes from one chunk's [D][64] tile to the next chunk's
+  ScanBlocks<true> kb(knP + cb * (D * CH), tile, n), wb(WT + cb * (D * CH), tile, n);
+  ScanBlocks<true> lb(dvlT + cb * (D * CH) + v0 * CH, tile, n), xb(XT + cb * (D * D) + v0 * D, 2 * tile, n);
+  ScanBlocks<true> sb(dhS + cb * (D * D) + slice * (D * 16), 2 * tile, n);
+  ScanBlocks<true> nb(dVnS + cb * (CH * D) + slice * (CH * 16), tile, n);
+  // per-lane parts of the addresses, the same for every chunk (bytes of global memory;
+  // elements of LDS)
+  const int q = (lane >> 2) & 3, p = lane & 3, from = tile_source(lane);
+  const int f_off = 4096 * wave + 16 * lane;                        // fragments (wave, j) of Kn, (wave, m, b) of -W^T
+  const int l_off = (4 * q4 + q) * CH * 2 + 32 * wave + 8 * p;      // dv_local^T row 4 q4 + q, t = 16 wave + 4 p ..
+  const int x_off = (4 * q4 + q) * D * 2 + 64 * wave + 16 * p;      // X^T row 4 q4 + q, k = 32 wave + 8 p ..
+  const int s_own = r * SCAN_SROW + 32 * wave + 8 * q4;
+  const int v_own = r * SCAN_VROW + 32 * (wave >> 1) + 8 * q4 + 4 * (wave & 1), v_in = r * SCAN_VROW + 8 * q4;
+  // the outputs, read transposed: dS [k][16] rows 32 wave .., dVn [t][16] rows 16 wave ..
+  const E* v_tr = Vx + (4 * q4 + (r >> 2)) * SCAN_VROW + 32 * (wave >> 1) + 8 * (r & 3) + 4 * (wave & 1);
+  const int s_out = ((32 * wave + 16 * (q4 >> 1) + r) * 16 + 8 * (q4 & 1)) * 2, v_out = ((16 * wave + r) * 16 + 4 * q4) * 2;
+  X8 fn[SCAN_DEPTH][4], fw[SCAN_DEPTH][2][2], fx[SCAN_DEPTH], x;
+  X4 fl[SCAN_DEPTH], dvl;
+  float gl[SCAN_DEPTH];
+  // l: the step's place after the table's and the blocks' first
+  auto issue_n = [&](int slot, int l) __attribute__((always_inline)) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) kofs[j] = 2 * (r * 128 + 8 * ((4 * j + q4) ^ r));
+    for (int j = 0; j < 4; ++j) fn[slot][j] = buf_ld16<X8>(kb.buffer(), f_off, kb.offset(l) + 1024 * ((wave + j) & 3));
+    fl[slot] = buf_ld8<X4>(lb.buffer(), l_off, lb.offset(l));
+    fx[slot] = buf_ld16<X8>(xb.buffer(), x_off, xb.offset(l));
+    gl[slot] = tab.glast(l);
+  };
+  auto issue_w = [&](int slot, int l) __attribute__((always_inline)) {
 #pragma unroll
-    for (int j = 0; j < 2; ++j) wofs[j] = 2 * (r * 64 + 8 * ((4 * j + q4) ^ ((r >> 1) & 7)));
+    for (int m = 0; m < 2; ++m)
 #pragma unroll
-    for (int i4 = 0; i4 < 4; ++i4) dofs[i4] = 2 * (r * 64 + 8 * ((2 * i4 + (q4 >> 1)) ^ ((r >> 1) & 7)) + 4 * (q4 & 1));
+      for (int b = 0; b < 2; ++b) fw[slot][m][b] = buf_ld16<X8>(wb.buffer(), f_off + 2048 * m + 1024 * b, wb.offset(l));
+  };
+  auto next_inputs = [&](int slot) __attribute__((always_inline)) {
+    dvl = tile_exchange(fl[slot], from);
+    x = tile_exchange(fx[slot], from);
+  };
+  X8 own = to8<E>(f32x8{});
+  st8(Sx + s_own, own);
 #pragma unroll
-    for (int m = 0; m < 8; ++m) xofs[m] = 2 * (r * 128 + 8 * ((2 * m + (q4 >> 1)) ^ r) + 4 * (q4 & 1));
-    const int sofs = 2 * (r * BS_SROW + 4 * q4), vofs = 2 * (r * BS_VROW + 4 * q4);
-    for (int tau = -BS_DEPTH; tau < n; ++tau) {
-      if (tau >= 0) {
-        char* base = reinterpret_cast<char*>(&stage[tau & (BS_STAGES - 1)]);
-        const char* knb = base + offsetof(BwdStage<E>, kn);
-        const char* wtb = base + offsetof(BwdStage<E>, wt);
-        const char* dvb = base + offsetof(BwdStage<E>, dvl);
-        const char* xtb = base + offsetof(BwdStage<E>, xt);
-        // every operand read is issued ahead of the MFMAs that use them (the
-        // kdec Kn fragments first); the scheduling barriers keep the compiler
-        // from interleaving them one by one
-        X8 fk[4][4], fw[8][2];
-        f32x4 xv[8];
+  for (int i = 0; i < SCAN_DEPTH; ++i) {
+    issue_n(i, i);
+    issue_w(i, i);
+  }
+  kb.advance();
+  wb.advance();
+  lb.advance();
+  xb.advance();
+  float g_now = __expf(gl[0]);
+  next_inputs(0);
+  lds_barrier();
+  auto step = [&](auto place, auto more) __attribute__((always_inline)) {
+    constexpr int s = decltype(place)::value;
+    // dVn = dv_local + (kdec Kn) dS_{c+1}, this wave's own block of k first
+    f32x4 acc = mfma(fn[s][0], own, cvtf4(dvl));
+    X8 sx[3];
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
+    for (int j = 1; j < 4; ++j) sx[j - 1] = ld8(Sx + r * SCAN_SROW + 32 * ((wave + j) & 3) + 8 * q4);
+    const X8 ds_out = ld8_tr16(Sx, SCAN_SROW, 32 * wave);
 #pragma unroll
-          for (int i4 = 0; i4 < 4; ++i4) fk[i4][j] = *reinterpret_cast<const X8*>(knb + kofs[j] + 4096 * i4);
-        // dVn = dv_local + (kdec Kn) dS_{c+1}, accumulated onto dv_local
-        f32x4 dv[4];
+    for (int j = 1; j < 4; ++j) acc = mfma(fn[s][j], sx[j - 1], acc);
+    buf_st16<OUT>(sb.buffer(), s_out + sb.offset(s), ds_out);
+    // the first two terms of dS_c = exp(G_last) dS_{c+1} + X + (-W^T) dVn
+    const f32x8 xf = cvtf8(x);
 #pragma unroll
-        for (int i4 = 0; i4 < 4; ++i4) dv[i4] = cvtf4(*reinterpret_cast<const X4*>(dvb + dofs[i4]));
-        const float glast = reinterpret_cast<const BwdStage<E>*>(base)->glast;
+    for (int m = 0; m < 2; ++m)
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
+      for (int i = 0; i < 4; ++i) dS[m][i] = dS[m][i] * g_now + xf[4 * m + i];
+    *reinterpret_cast<X4*>(Vx + v_own) = to4<E>(acc);
+    lds_barrier();
+    const X8 b0 = ld8(Vx + v_in), b1 = ld8(Vx + v_in + 32);
+    typedef __attribute__((address_space(3))) i16x4 lds_i16x4;
+    const X4 dv_out = __builtin_bit_cast(X4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)v_tr));
+    constexpr int next = (s + 1) % SCAN_DEPTH;
+    g_now = __expf(gl[next]);
+    next_inputs(next);
+    if constexpr (decltype(more)::value) issue_n(s, s);
 #pragma unroll
-          for (int m = 0; m < 8; ++m) fw[m][j] = *reinterpret_cast<const X8*>(wtb + wofs[j] + 2048 * m);
+    for (int m = 0; m < 2; ++m) dS[m] = mfma(fw[s][m][0], b0, dS[m]);
 #pragma unroll
-        for (int m = 0; m < 8; ++m) xv[m] = cvtf4(*reinterpret_cast<const X4*>(xtb + xofs[m]));
-        __builtin_amdgcn_sched_barrier(0);
-        X4 sh[8];
-#pragma unroll
-        for (int m = 0; m < 8; ++m) sh[m] = to4<E>(dS[m]);
-        // beside it, the first two terms of dS_c = exp(G_last) dS_{c+1} + X + (-W^T) dVn
-        const float gC = __expf(glast);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const X8 sb = cat(sh[2 * j], sh[2 * j + 1]);
-#pragma unroll
-          for (int i4 = 0; i4 < 4; ++i4) dv[i4] = mfma(fk[i4][j], sb, dv[i4]);
-#pragma unroll
-          for (int m = 2 * j; m < 2 * j + 2; ++m) dS[m] = dS[m] * gC + xv[m];
-        }
-        __builtin_amdgcn_sched_barrier(0);
-        // the -W^T fragments have been read (a wave's LDS operations complete in
-        // order): the -W^T region now takes this step's outputs
-        char* sb = base + offsetof(BwdStage<E>, wt);
-#pragma unroll
-        for (int m = 0; m < 8; ++m) *reinterpret_cast<X4*>(sb + sofs + 32 * m) = sh[m];
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-          const X8 nb = pack_permv<E>(dv[2 * j], dv[2 * j + 1]);
-#pragma unroll
-          for (int m = 0; m < 8; ++m) dS[m] = mfma(fw[m][j], nb, dS[m]);
-        }
-        char* vbp = sb + sizeof(BwdScratch<E>::s);
-#pragma unroll
-        for (int i4 = 0; i4 < 4; ++i4) *reinterpret_cast<X4*>(vbp + vofs + 32 * i4) = to4<E>(dv[i4]);
-      }
-      lds_barrier();
+    for (int m = 0; m < 2; ++m) dS[m] = mfma(fw[s][m][1], b1, dS[m]);
+    if constexpr (decltype(more)::value) issue_w(s, s);
+    buf_st8<OUT>(nb.buffer(), v_out, nb.offset(s), dv_out);
+    own = to8<E>(f32x8{dS[0][0], dS[0][1], dS[0][2], dS[0][3], dS[1][0], dS[1][1], dS[1][2], dS[1][3]});
+    st8(Sx + s_own, own);
+    if constexpr (SC1 && decltype(more)::value) {
+      // the stores of BWD_ANNOUNCE steps ago have completed: that many full steps were issued after them
+      asm volatile("" ::: "memory");
+      wait_vmem_le<BWD_ANNOUNCE * BWD_STEP_OPS>();
     }
-  } else {
-    // Step tau, both loaders: wait for their part of step tau+1's chunk, then
-    // refill stage (tau-1)%4 with their part of step tau+3's chunk (loader 1
-    // first stores step tau-1's outputs from that stage's -W^T region).  Loads
-    // and stores retire in issue order, so a loader waits by letting exactly
-    // the operations it issued after that part stay in flight (as in the
-    // forward scan).  Loader 1's wait at step tau >= 3 also covers the copy-out
-    // of step tau-3 (issued before step tau+1's part), so with a bwd_dkw beside
-    // the scan it then announces that step's chunk: one atomic add, in flight
-    // with the step's other operations and counted in the next wait.
-    const int j = wave - 1;
-    for (int tau = -BS_DEPTH; tau < n; ++tau) {
-      const int xn = tau + 1, xo = tau - 1, xi = tau + BS_DEPTH;
-      if (xn >= 0 && xn < n) {
-        const bool later = xn + 1 < n;  // this loader's part of step tau+2's chunk is in flight
-        if (j == 0) {
-          if (later)
-            wait_vmem_le<BWD_PART_COPIES[0]>();
-          else
-            wait_vmem_all();
-          bwd_fix_tail(stage[xn & (BS_STAGES - 1)], chunks, c_end - 1 - xn, lane);
-        } else {
-          const bool stored = tau >= 2;                 // the copy-out of step tau-2 came after this part
-          const bool announced = ready && tau >= 4;     // and step tau-1's announcement (of step tau-4)
-          if (later && announced)
-            wait_vmem_le<BWD_PART_COPIES[1] + BWD_OUT_STORES + 1>();
-          else if (later && stored)
-            wait_vmem_le<BWD_PART_COPIES[1] + BWD_OUT_STORES>();
-          else if (later)
-            wait_vmem_le<BWD_PART_COPIES[1]>();
-          else if (announced)
-            wait_vmem_le<BWD_OUT_STORES + 1>();
-          else if (stored)
-            wait_vmem_le<BWD_OUT_STORES>();
-          else
-            wait_vmem_all();
-          if (ready && tau >= 3) bwd_publish(ready, c_end - 1 - (tau - 3), H, h, lane);
-        }
+    lds_barrier();
+  };
+  int announced = 0;  // steps whose chunks are announced
+  auto round = [&](int tau, auto first) __attribute__((always_inline)) {
+    tab.advance(tau + SCAN_DEPTH);
+    auto announced_step = [&](auto place) __attribute__((always_inline)) {
+      step(place, Int<1>());
+      // every wave has waited for its stores of step tau + place - BWD_ANNOUNCE
+      if constexpr (SC1 && (!decltype(first)::value || decltype(place)::value >= BWD_ANNOUNCE)) {
+        if (wave == 0) bwd_publish(ready, c_last - announced, H, h, lane);
+        ++announced;
       }
-      if (j == 1 && xo >= 0) {
-        if (ready)
-          bwd_copy_out<true>(bwd_scratch(stage[xo & (BS_STAGES - 1)]), c_end - 1 - xo, H, h, slice, lane, dhS, dVnS);
-        else
-          bwd_copy_out<false>(bwd_scratch(stage[xo & (BS_STAGES - 1)]), c_end - 1 - xo, H, h, slice, lane, dhS, dVnS);
-      }
-      if (xi < n)
-        bwd_issue(stage[xi & (BS_STAGES - 1)], chunks, c_end - 1 - xi, H, h, v0, lane, j, knP, gc, dvlT, XT, WT);
-      lds_barrier();
-    }
-    if (n > 0 && j == 1) {
-      if (ready)
-        bwd_copy_out<true>(bwd_scratch(stage[(n - 1) & (BS_STAGES - 1)]), c_end - n, H, h, slice, lane, dhS, dVnS);
-      else
-        bwd_copy_out<false>(bwd_scratch(stage[(n - 1) & (BS_STAGES - 1)]), c_end - n, H, h, slice, lane, dhS, dVnS);
-      if (ready) {
-        // the loop announced steps 0 .. n-5; the rest once every store has completed
-        wait_vmem_all();
-        for (int s = max(n - 4, 0); s < n; ++s) bwd_publish(ready, c_end - 1 - s, H, h, lane);
-      }
-    }
+    };
+    announced_step(Int<0>());
+    announced_step(Int<1>());
+    announced_step(Int<2>());
+    announced_step(Int<3>());
+    kb.advance();
+    wb.advance();
+    lb.advance();
+    xb.advance();
+    sb.advance();
+    nb.advance();
+  };
+  int tau = 0;
+  if (n >= SCAN_DEPTH) {
+    round(0, Int<1>());
+    for (tau = SCAN_DEPTH; tau + SCAN_DEPTH <= n; tau += SCAN_DEPTH) round(tau, Int<0>());
+  }
+  if (tau < n) step(Int<0>(), Int<0>());
+  if (tau + 1 < n) step(Int<1>(), Int<0>());
+  if (tau + 2 < n) step(Int<2>(), Int<0>());
+  if constexpr (SC1) {
+    wait_vmem_all();
+    lds_barrier();
+    if (wave == 0)
+      for (; announced < n; ++announced) bwd_publish(ready, c_last - announced, H, h, lane);
   }
 }
 
@@ -1297,9 +1199,9 @@ static hipError_t launch_bwd_t(const BwdArgs& a, hipStream_t stream) {
   }
   {
     TimedLaunch tl(K_BWD_SCAN, stream);
-    hipLaunchKernelGGL(bwd_scan_kernel<E>, dim3(a.H * (D / 16), a.n_docs), dim3(BS_THREADS), 0, stream, B(B_KNP),
-                       Ff(F_GC), B(B_DVLT), B(B_XT), B(B_WT), a.chunks, a.doc_chunk, a.H, B(B_DH), B(B_DVN),
-                       beside ? ready : nullptr, beside ? resident : nullptr);
+    const auto kernel = beside ? bwd_scan_kernel<E, true> : bwd_scan_kernel<E, false>;
+    hipLaunchKernelGGL(kernel, dim3(a.H * (D / 16), a.n_docs), dim3(SCAN_THREADS), 0, stream, B(B_KNP), Ff(F_GC),
+                       B(B_DVLT), B(B_XT), B(B_WT), a.chunks, a.doc_chunk, a.H, B(B_DH), B(B_DVN), ready, resident);
   }
   if (beside) {
     launch_resident_gate(resident, a.H * (D / 16) * a.n_docs, a.side);

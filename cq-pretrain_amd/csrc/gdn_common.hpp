@@ -20,6 +20,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 namespace cqgdn {
 
 constexpr int D = 128;   // head dimension (d_k = d_v), the only one the reference accepts
@@ -58,29 +60,15 @@ __device__ __forceinline__ f32x4 cvtf4(bf16x4 x) { return __builtin_convertvecto
 __device__ __forceinline__ f32x8 cvtf8(bf16x8 x) { return __builtin_convertvector(x, f32x8); }
 __device__ __forceinline__ bf16x8 cvt8(f32x8 x) { return __builtin_convertvector(x, bf16x8); }
 
-// Two C tiles (rows m0..m0+15 and m0+16..m0+31 of one column) -> one operand
-// in the permuted slot map.
-__device__ __forceinline__ bf16x8 pack_perm(f32x4 lo, f32x4 hi) {
-  f32x8 x = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-  return cvt8(x);
-}
-
 __device__ __forceinline__ bf16x8 cat(bf16x4 a, bf16x4 b) {
   return __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7);
-}
-
-__device__ __forceinline__ bf16x8 neg8(bf16x8 x) {
-  // flip the sign bits (exact)
-  u32x4 u = __builtin_bit_cast(u32x4, x);
-  u ^= 0x80008000u;
-  return __builtin_bit_cast(bf16x8, u);
 }
 
 // Storage order that makes a permuted-map fragment one contiguous 16-byte
 // load: within every 32-element block, logical index x = 4q + s' + 16h
 // (q = 0..3, s' = 0..3, h = 0..1) is stored at 8q + 4h + s'.  Tensors that
-// are only ever read as permuted-map operands (W, KgT, W^T, the scan copy of
-// Kn) are written in this order, so their consumers use ld8 at 32j + 8*q4.
+// are only ever read as permuted-map operands (W rows; the event runs of KgT and
+// -W^T) are written in this order.
 __host__ __device__ __forceinline__ int perm32(int x) {
   return (x & ~31) | (((x >> 2) & 3) << 3) | (((x >> 4) & 1) << 2) | (x & 3);
 }
@@ -95,21 +83,6 @@ __device__ __forceinline__ bf16x4 ld4(const bf16* p) { return *reinterpret_cast<
 __device__ __forceinline__ bf16x8 ld8_nt(const bf16* p) {
   return __builtin_nontemporal_load(reinterpret_cast<const bf16x8*>(p));
 }
-// 16 bytes stored with the non-temporal hint: for whole rows written while the
-// caches hold data the same kernel has yet to read.
-__device__ __forceinline__ void st8_nt(bf16* p, bf16x8 x) {
-  __builtin_nontemporal_store(x, reinterpret_cast<bf16x8*>(p));
-}
-// permuted map, k-contiguous storage: p points at element k0 + 4*q4
-__device__ __forceinline__ bf16x8 ld8p(const bf16* p) { return cat(ld4(p), ld4(p + 16)); }
-// natural map, strided storage: element s at p[s * stride]
-__device__ __forceinline__ bf16x8 ld8s(const bf16* p, int stride) {
-  bf16x8 x;
-#pragma unroll
-  for (int s = 0; s < 8; ++s) x[s] = p[s * stride];
-  return x;
-}
-
 __device__ __forceinline__ void st4(bf16* p, f32x4 x) { *reinterpret_cast<bf16x4*>(p) = cvt4(x); }
 __device__ __forceinline__ void st8(bf16* p, bf16x8 x) { *reinterpret_cast<bf16x8*>(p) = x; }
 
@@ -199,7 +172,8 @@ template <class E>
 __device__ __forceinline__ typename Vec<E>::x8 scaled8(bf16x8 x, float r) {
   return to8<E>(cvtf8(x) * r);
 }
-// two C tiles -> one permuted-map operand (as pack_perm, for either element type)
+// Two C tiles (rows m0..m0+15 and m0+16..m0+31 of one column) -> one operand
+// in the permuted slot map.
 template <class E>
 __device__ __forceinline__ typename Vec<E>::x8 pack_permv(f32x4 lo, f32x4 hi) {
   return to8<E>(f32x8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]});
@@ -244,9 +218,6 @@ __device__ __forceinline__ f16x8 ld8_trp(const f16* tile, int ld, int k0, int n0
 }
 __device__ __forceinline__ f16x8 ld8_nt(const f16* p) {
   return __builtin_nontemporal_load(reinterpret_cast<const f16x8*>(p));
-}
-__device__ __forceinline__ void st8_nt(f16* p, f16x8 x) {
-  __builtin_nontemporal_store(x, reinterpret_cast<f16x8*>(p));
 }
 template <class E>
 __device__ __forceinline__ typename Vec<E>::x8 scaled8(f16x8 x, float r) {
@@ -316,9 +287,6 @@ __device__ __forceinline__ bf16x8 col8_combine(const Col8& g) {
   }
   return __builtin_bit_cast(bf16x8, out);
 }
-__device__ __forceinline__ bf16x8 gather8_col_rows(const bf16* M, int ld, int row0, int col0, int nrows) {
-  return col8_combine(col8_load_rows(M, ld, row0, col0, nrows));
-}
 // The same gathers over an fp16 matrix (they move 16-bit values without looking at them)
 __device__ __forceinline__ Col8 col8_load(const f16* M, int ld, int row0, int col0) {
   return col8_load(reinterpret_cast<const bf16*>(M), ld, row0, col0);
@@ -349,78 +317,6 @@ template <int N>
 __device__ __forceinline__ void wait_vmem_le() {
   static_assert(N >= 0 && N < 64, "vmcnt is 6 bits");
   __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 15) | ((N >> 4) << 14));
-}
-
-// vmcnt(parts * P + stores * S) for counts known only at run time (parts and
-// stores in 0..2): the wait of a wave that has issued `parts` copy parts of P
-// operations and `stores` store groups of S since the operations it waits for.
-template <int P, int S>
-__device__ __forceinline__ void wait_vmem_parts(int parts, int stores) {
-  static_assert(2 * P + 2 * S < 64, "vmcnt is 6 bits");
-  switch (parts * 3 + stores) {
-    case 0: wait_vmem_le<0>(); break;
-    case 1: wait_vmem_le<S>(); break;
-    case 2: wait_vmem_le<2 * S>(); break;
-    case 3: wait_vmem_le<P>(); break;
-    case 4: wait_vmem_le<P + S>(); break;
-    case 5: wait_vmem_le<P + 2 * S>(); break;
-    case 6: wait_vmem_le<2 * P>(); break;
-    case 7: wait_vmem_le<2 * P + S>(); break;
-    default: wait_vmem_le<2 * P + 2 * S>(); break;
-  }
-}
-
-// Hand-off counters in LDS between the waves of one workgroup, in place of
-// s_barrier: a producer wave publishes a count once everything it covers is in
-// LDS (its own LDS operations complete in order, and an asynchronous copy has
-// landed once vmcnt says so); a consumer wave polls the count.  Every wait is
-// bounded: after FLAG_SPIN_LIMIT polls it gives up and returns false, so a
-// broken hand-off ends the kernel with wrong results instead of hanging it.
-// The casts name the LDS address space: through a plain volatile pointer the
-// accesses would become flat operations that wait for every vector memory
-// operation in flight (a loader's own copies included).
-constexpr int FLAG_SPIN_LIMIT = 1 << 20;
-typedef __attribute__((address_space(3))) volatile int lds_vint;
-typedef __attribute__((address_space(3))) volatile long long lds_vi64;
-__device__ __forceinline__ int lds_flag_read(const int* f) {
-  return __builtin_amdgcn_readfirstlane(*(lds_vint*)(f));
-}
-__device__ __forceinline__ void lds_flag_publish(int* f, int v) {
-  asm volatile("" ::: "memory");
-  *(lds_vint*)(f) = v;
-  asm volatile("" ::: "memory");
-}
-// two adjacent counts in one LDS read
-__device__ __forceinline__ int2 lds_flag_read2(const int* f) {
-  const long long v = *(lds_vi64*)(f);
-  return int2{(int)v, (int)(v >> 32)};
-}
-template <bool SLEEP>
-__device__ __forceinline__ bool lds_flag_wait_ge(const int* f, int target) {
-  for (int i = 0; i < FLAG_SPIN_LIMIT; ++i) {
-    if (lds_flag_read(f) >= target) {
-      asm volatile("" ::: "memory");
-      return true;
-    }
-    if (SLEEP) __builtin_amdgcn_s_sleep(1);
-  }
-  return false;
-}
-
-// A scan consumer's wait for step target-1 from both of its loaders (counts
-// flags[0], flags[1]); `seen` gets the smaller count read.  Bounded (see
-// lds_flag_wait_ge): false if it gave up.
-__device__ __forceinline__ bool scan_wait_ready(const int* flags, int target, int& seen) {
-  for (int i = 0; i < FLAG_SPIN_LIMIT; ++i) {
-    const int2 v = lds_flag_read2(flags);
-    const int mn = min(__builtin_amdgcn_readfirstlane(v.x), __builtin_amdgcn_readfirstlane(v.y));
-    if (mn >= target) {
-      asm volatile("" ::: "memory");
-      seen = mn;
-      return true;
-    }
-  }
-  return false;
 }
 
 typedef __attribute__((address_space(3))) void* lds_void_ptr;
@@ -593,9 +489,12 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t buf_rsrc(const void* base, int
 __device__ __forceinline__ void buf_stf(__amdgpu_buffer_rsrc_t rs, int voff, int soff, float x) {
   __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, x), rs, voff, soff, 0);
 }
-template <class X8>
-__device__ __forceinline__ void buf_st16(__amdgpu_buffer_rsrc_t rs, int voff, int soff, X8 x) {
-  __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, x), rs, voff, soff, 0);
+// 16 bytes.  No scalar offset: a store of more than 8 bytes reads its last two registers
+// a cycle late, and the compiler keeps the next instruction off them only if the store has
+// no scalar offset (with one, a v_lshlrev right after a store changed what it stored).
+template <int CPOL = 0, class X8>
+__device__ __forceinline__ void buf_st16(__amdgpu_buffer_rsrc_t rs, int voff, X8 x) {
+  __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, x), rs, voff, 0, CPOL);
 }
 __device__ __forceinline__ void buf_st1(__amdgpu_buffer_rsrc_t rs, int voff, int soff, float x) {
   __builtin_amdgcn_raw_buffer_store_b16(__builtin_bit_cast(unsigned short, (bf16)x), rs, voff, soff, 0);
@@ -606,6 +505,18 @@ __device__ __forceinline__ void buf_st4(__amdgpu_buffer_rsrc_t rs, int voff, int
   __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, to4<E>(x)), rs, voff, soff, 0);
 }
 
+template <class X8>
+__device__ __forceinline__ X8 buf_ld16(__amdgpu_buffer_rsrc_t rs, int voff, int soff) {
+  return __builtin_bit_cast(X8, __builtin_amdgcn_raw_buffer_load_b128(rs, voff, soff, 0));
+}
+template <class X4>
+__device__ __forceinline__ X4 buf_ld8(__amdgpu_buffer_rsrc_t rs, int voff, int soff) {
+  return __builtin_bit_cast(X4, __builtin_amdgcn_raw_buffer_load_b64(rs, voff, soff, 0));
+}
+template <int CPOL = 0, class X4>
+__device__ __forceinline__ void buf_st8(__amdgpu_buffer_rsrc_t rs, int voff, int soff, X4 x) {  // 8 bytes
+  __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, x), rs, voff, soff, CPOL);
+}
 // ---- hand-off between two kernels running at the same time ----------------
 // The eight XCDs' L2 caches are not coherent with one another.  Data that one
 // running kernel hands to another is stored and loaded with the cache-policy bit
@@ -621,11 +532,6 @@ __device__ __forceinline__ void dma16_sc1(const void* src, void* lds) {
 template <class X8>
 __device__ __forceinline__ X8 buf_ld16_sc1(__amdgpu_buffer_rsrc_t rs, int voff) {
   return __builtin_bit_cast(X8, __builtin_amdgcn_raw_buffer_load_b128(rs, voff, 0, CPOL_SC1));
-}
-// 16 bytes stored at device scope with the non-temporal hint
-template <class X8>
-__device__ __forceinline__ void buf_st16_nt_sc1(__amdgpu_buffer_rsrc_t rs, int voff, X8 x) {
-  __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, x), rs, voff, 0, CPOL_NT | CPOL_SC1);
 }
 __device__ __forceinline__ void count_add(int* p) {
   __hip_atomic_fetch_add(p, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -657,6 +563,130 @@ struct ChunkInfo {
 };
 __device__ __forceinline__ ChunkInfo chunk_info(const int32_t* table, int c) {
   return ChunkInfo{table[2 * c], table[2 * c + 1]};
+}
+
+// ---- the state scans --------------------------------------------------------
+constexpr int SCAN_THREADS = 256;
+constexpr int SCAN_DEPTH = 4;    // chunks whose operands are in flight or in registers
+constexpr int SCAN_SROW = 136;   // row stride (elements) of the state's [v][k] exchange tile
+constexpr int SCAN_VROW = 72;    // row stride (elements) of the [v][t] exchange tile
+
+// What a scan needs to know of the chunks it requests: where their event rows are (the
+// rows of head h of an [events][H][128] tensor, as a raw buffer that ends after the
+// chunk's last row, so that rows past it read as zeros) and G of their last event.  A
+// round of SCAN_DEPTH steps looks up steps x .. x + SCAN_DEPTH (one more than a round:
+// the first operand is requested a step early), held in lanes 0 .. SCAN_DEPTH, and a
+// step's entry is a few v_readlane.  Each round requests the chunk table entries of two
+// rounds on and the gates of the next (whose rows the entries requested a round before
+// give), so no step waits for them, and without a branch, so that the compiler can count
+// the requests in flight.  Step x is chunk first + sign * x; the rows of steps past the
+// last are empty.
+class ScanTable {
+ public:
+  // the entries of steps 0 .. SCAN_DEPTH
+  __device__ __forceinline__ ScanTable(const int32_t* chunks, const float* gc, const void* rows, int first, int sign,
+                                       int n, int H, int h, int lane)
+      : chunks_(chunks), gc_(gc + h), rows_(reinterpret_cast<uint64_t>(rows) + (uint64_t)h * D * 2), first_(first),
+        sign_(sign), n_(n), H_(H), at_(min(lane, SCAN_DEPTH)) {
+    ChunkInfo now = info(0);
+    next_ = info(SCAN_DEPTH);
+    after_ = info(2 * SCAN_DEPTH);
+    gate_ = gate(now);
+    next_gate_ = gate(next_);
+    locate(now, 0);
+  }
+  // on to the entries of steps x .. x + SCAN_DEPTH
+  __device__ __forceinline__ void advance(int x) {
+    locate(next_, x);
+    gate_ = next_gate_;
+    next_ = after_;
+    next_gate_ = gate(next_);
+    after_ = info(x + 2 * SCAN_DEPTH);
+  }
+  // of step x + l
+  __device__ __forceinline__ __amdgpu_buffer_rsrc_t rows(int l) const {
+    const uint64_t at = (uint64_t)(uint32_t)__builtin_amdgcn_readlane(lo_, l) |
+                        (uint64_t)(uint32_t)__builtin_amdgcn_readlane(hi_, l) << 32;
+    return buf_rsrc(reinterpret_cast<const void*>(at), __builtin_amdgcn_readlane(bytes_, l));
+  }
+  __device__ __forceinline__ float glast(int l) const {
+    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, gate_), l));
+  }
+
+ private:
+  __device__ __forceinline__ ChunkInfo info(int x) const {
+    return chunk_info(chunks_, first_ + sign_ * min(x + at_, n_ - 1));
+  }
+  __device__ __forceinline__ float gate(ChunkInfo c) const { return gc_[(size_t)(c.start + c.len - 1) * H_]; }
+  __device__ __forceinline__ void locate(ChunkInfo c, int x) {
+    const uint64_t at = rows_ + (uint64_t)((size_t)c.start * H_) * (D * 2);
+    lo_ = (int)(uint32_t)at;
+    hi_ = (int)(uint32_t)(at >> 32);
+    bytes_ = x + at_ < n_ ? ((c.len - 1) * H_ + 1) * D * 2 : 0;
+  }
+  const int32_t* chunks_;
+  const float* gc_;
+  uint64_t rows_;
+  int first_, sign_, n_, H_, at_;
+  int lo_, hi_, bytes_;
+  ChunkInfo next_, after_;
+  float gate_, next_gate_;
+};
+
+// One head's block of a [chunks][H][..] buffer over the steps of a scan (REVERSE: from
+// the last chunk down): a round's chunks are reached from one raw buffer with the
+// step's place in the round as a scalar offset, so a step computes no address.  Steps
+// past the last lie past the buffer's end: loads return zeros.
+template <bool REVERSE>
+class ScanBlocks {
+ public:
+  // first: the block of step 0; size: bytes from a chunk's block to the next chunk's; n: steps
+  __device__ __forceinline__ ScanBlocks(const void* first, int64_t size, int n)
+      : at_(reinterpret_cast<uint64_t>(first) - (REVERSE ? SCAN_DEPTH * size : 0)), size_(size), left_(n) {}
+  __device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer() const {
+    return buf_rsrc(reinterpret_cast<const void*>(at_), (SCAN_DEPTH + 1) * (int)size_);
+  }
+  __device__ __forceinline__ int offset(int l) const {
+    return (l < left_ ? (REVERSE ? SCAN_DEPTH - l : l) : SCAN_DEPTH + 1) * (int)size_;
+  }
+  __device__ __forceinline__ void advance() {
+    at_ += (REVERSE ? -SCAN_DEPTH : SCAN_DEPTH) * size_;
+    left_ -= SCAN_DEPTH;
+  }
+
+ private:
+  uint64_t at_;
+  int64_t size_;
+  int left_;
+};
+
+// a number as a type, for the scans' unrolled steps
+template <int N>
+using Int = std::integral_constant<int, N>;
+
+// The vector memory unit takes the 64 lanes of a load or store four at a time: a quad
+// whose lanes fall in one 128-byte line passes in one go, one whose lanes fall in four
+// lines in four.  Measured on one CU (four waves, operands in L2): 16 bytes a lane with
+// whole quads of a row 9.2 ns per KB, with lane r % 16 on row r (an MFMA fragment read
+// straight from a row-major matrix) 28.5; 8 bytes a lane 14.6 against 54.7; stores 24
+// against 61.  So what a scan reads is either stored fragment by fragment (its lanes'
+// 16 bytes in lane order), or copied to LDS by whole rows, or read by quads and brought to
+// the MFMA layout by the exchange below.
+//
+// x of lane 16 q + 4 p + g at lane 16 g + 4 q + p: a 16-row tile read by quads (lane
+// 16 g + 4 q + p holds piece p of row 4 g + q) to the MFMA result's layout (piece g of
+// row 4 q + p).  `from` = 4 * the source lane.
+__device__ __forceinline__ int tile_source(int lane) {
+  return 4 * (16 * ((lane >> 2) & 3) + 4 * (lane & 3) + (lane >> 4));
+}
+template <class X>  // 8 or 16 bytes
+__device__ __forceinline__ X tile_exchange(X x, int from) {
+  typedef int words __attribute__((ext_vector_type(sizeof(X) / 4)));
+  words w = __builtin_bit_cast(words, x);
+  asm volatile("" : "+v"(w));  // keeps its place between the barriers (it would be hoisted, and wait for x there)
+#pragma unroll
+  for (unsigned i = 0; i < sizeof(X) / 4; ++i) w[i] = __builtin_amdgcn_ds_bpermute(from, w[i]);
+  return __builtin_bit_cast(X, w);
 }
 
 // The (head, chunk position) of this workgroup in a grid of (H, NC) chunk-heads.

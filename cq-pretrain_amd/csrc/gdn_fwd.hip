@@ -12,7 +12,7 @@
 // Kernels:
 //   fwd_prep   grid (NC, H), 4 waves: l2norm q,k; cumsum g; A via MFMA; the unit
 //              lower-triangular inverse in LDS (fp32); W, W^T, U via MFMA.
-//   fwd_state  grid (H * 8 value slices, docs), 1 wave: the serial scan, a 128x16
+//   fwd_scan   grid (H * 8 value slices, docs), 4 waves: the serial scan, a 128x16
 //              fp32 state slice held in registers across all chunks of a document.
 //   fwd_out    grid (NC, H), 4 waves: O^T = gam * (h^T Qn^T) + Vn^T P^T, all MFMA.
 #include "gdn_common.hpp"
@@ -270,18 +270,23 @@ __global__ __launch_bounds__(256, 3) void fwd_prep_kernel(
     }
   }
 
-  // Kg^T tile [k][perm32(t)] over the solve's matrix (free now), stored below.
-  // Row k's columns are XORed with 16 ((k / 8) % 4) (16-byte blocks stay whole):
-  // the four threads of event t write rows 8 apart, which then fall in disjoint
-  // banks instead of one.
+  // Kg^T over the solve's matrix (free now), in the order the scan reads it (stored
+  // below): fragment (k / 16, t / 32), and in it 16-byte granule 16 g + r holding row
+  // k = 16 (k / 16) + r at the four-runs g of both halves of the 32 events (perm32).  A
+  // granule's low three bits are XORed with g + 4 (r / 8): the 16 (event run, quarter)
+  // pairs that write together then spread over all the banks, and the reads stay
+  // conflict-free.
   E* kgs = reinterpret_cast<E*>(Af);
   static_assert(sizeof(Af) >= D * CH * sizeof(E), "the KgT tile must fit the solve matrix");
   {
-    const int t = tid >> 2, p = tid & 3, tp = perm32(t) ^ (16 * p);  // (k / 8) % 4 = p for k = 32 j + 8 p + s
+    const int t = tid >> 2, p = tid & 3, tp = perm32(t), g = (tp >> 3) & 3;
 #pragma unroll
     for (int j = 0; j < 4; ++j)
 #pragma unroll
-      for (int s = 0; s < 8; ++s) kgs[(32 * j + 8 * p + s) * CH + tp] = kg8[j][s];
+      for (int s = 0; s < 8; ++s) {
+        const int k = 32 * j + 8 * p + s, gran = 16 * g + ((k & 15) ^ (g + 4 * (p & 1)));
+        kgs[((2 * (k >> 4) + (t >> 5)) * 64 + gran) * 8 + (tp & 7)] = kg8[j][s];
+      }
   }
 
   // ---- W = T (beta gam K) -> W rows, U = T (beta V) -> U^T storage ----
@@ -337,355 +342,217 @@ __global__ __launch_bounds__(256, 3) void fwd_prep_kernel(
     E* kgt = KgT + cb * (D * CH);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const int seg = 256 * i + tid, kr = seg >> 3, part = seg & 7;
-      st8(kgt + kr * CH + 8 * part, ld8(kgs + kr * CH + 8 * (part ^ (2 * ((kr >> 3) & 3)))));
+      const int seg = 256 * i + tid;
+      st8(kgt + seg * 8, ld8(kgs + (seg ^ (((seg >> 4) & 3) + 4 * ((seg >> 3) & 1))) * 8));
     }
   }
   if (SCALED && blockIdx.x == 0 && blockIdx.y == 0 && tid == 0) vscale[0] = vs;
 }
 
 // ---------------------------------------------------------------------------
-// fwd_state: one wave per (head, 16-wide value slice, document)
+// fwd_scan: the serial scan, four waves per (head, 16-wide value slice, document)
 // ---------------------------------------------------------------------------
-// The scan is a chain of dependent chunk steps, so it runs at the speed one
-// step waits.  A workgroup serves one 16-wide value slice of one head with one
-// consumer wave (wave 0) and two loader waves.  Loaders copy each chunk's
-// operands global -> LDS asynchronously (global_load_lds) into a ring of
-// SC_STAGES stages.  Each chunk's copies are split between the two loaders
-// (issuing them is what bounds a step: a CU accepts about one 1 KB copy per
-// 20-30 cycles, so one wave issuing all 35 takes longer than the consumer's
-// MFMA work).  The consumer only reads LDS and writes its output tiles to LDS;
-// loader 1 stores them.  So no wave holds in-flight data in registers and the
-// consumer never waits on memory.
+// The scan is a chain of dependent chunk steps.  A workgroup serves one 16-wide value
+// slice of one head; wave w holds rows 32 w .. 32 w + 31 of the slice's fp32 state in two
+// C tiles and does a quarter of each contraction:
+//   v_new rows t = 16 w ..  = U + (-W rows) S      needs all of S, in the operand type
+//   S rows k = 32 w ..      = e^G S + Kg^T v_new   needs all of v_new
+// so a step passes the operand copy of S (4 KB) and v_new (2 KB) through LDS, with a
+// barrier after each, and its chain is 4 + 2 dependent MFMAs and two LDS round trips:
+// 48 us over 144 steps with no operand traffic.  (One wave doing it all needs 32 MFMAs in
+// a row and reads 34 KB of operands from LDS; with two loader waves feeding it the kernel
+// took 102 us.)
 //
-// The waves hand stages to each other through counts in LDS, not s_barrier:
-// a loader publishes a chunk once its part has landed, the consumer publishes
-// a chunk once it is done with it, and each wave waits only for the count it
-// needs.  With a barrier per step, every step lasted as long as the slower of
-// the consumer and the loaders plus the barrier; this way the loaders run up
-// to four chunks ahead and the two sides overlap.
+// What bounds a step now is what one CU's vector memory takes in: every workgroup of a
+// head reads all of -W and Kg^T, 34 KB a step, and writes 6 KB.  Each lane group has to
+// read whole 64-byte pieces for that (see "the vector memory unit" in gdn_common.hpp):
+//   Kg^T  is stored in fragment order by fwd_prep: 1 KB of contiguous lanes' operands a load;
+//   -W    rows go to LDS by asynchronous copies of four 256-byte rows (16-byte columns
+//         XOR-swizzled by row), each wave its own 16 rows, and come back as fragments;
+//   U^T   is read by quads and exchanged between lanes (tile_exchange);
+//   h^T, v_new^T leave as whole rows, read back from the LDS copies.
+// With fragments read straight from the row-major matrices the same kernel took 173 us.
+// Operands are requested SCAN_DEPTH steps ahead into registers (and four LDS rings);
+// 3, 5 or 6 steps measured the same.  No step computes an address (ScanBlocks, ScanTable)
+// and nothing in a round is conditional, so the compiler's own waits leave every later
+// request in flight; the first round is peeled because a loop entered with fewer
+// operations in flight than it runs with waits as strictly as its entry.
 //
-// LDS tiles are stored with 16-byte columns XOR-swizzled by row (chosen on the
-// source side of each copy), so the consumer's fragment reads, 16 rows at one
-// logical column, hit distinct banks:
-//   W   [64 rows t][16 cols]  col' = col ^ (t & 15)
-//   KgT [128 rows k][8 cols]  col' = col ^ ((k >> 1) & 7)
-//   U^T [16 rows v][8 cols]   col' = col ^ ((v >> 1) & 7)
-constexpr int SC_THREADS = 64 * 3;
-constexpr int SC_STAGES = 4;
-constexpr int SC_SROW = 136;  // scratch row stride (elements), S^T [v][k]
-constexpr int SC_VROW = 72;   // scratch row stride (elements), v_new^T [v][t]
-
+// Measured (H = 16, one document of 144 chunks / 15 documents, 520 chunks): 102.6 -> 86.0
+// us, 294 -> 247 us; 36 chunks 29.1 -> 23.7; four heads, 144 chunks 97.9 -> 75.3.  LDS
+// went from 136 KB to 72 KB a workgroup, so two share a CU.
+//
+// The waits for -W: loads, copies and stores of a wave retire in issue order, so a copy
+// has landed once at most as many operations are in flight as were surely issued after
+// it.  Counted are the operations of whole windows between barriers (the compiler may
+// reorder a window's own): a full step issues 11 (9 loads, 2 stores), and the store of
+// h^T precedes the wait.
+constexpr int FWD_STEP_OPS = 11, FWD_LOAD_OPS = 9;
 template <class E>
-struct __attribute__((aligned(16))) FwdStage {
-  E w[64 * 128];   // -W rows t
-  E kg[128 * 64];  // KgT rows k
-  E ut[16 * 64];   // U^T rows of the slice
-  float glast;     // G of the chunk's last event
-  float pad[3];
-};
-
-// the consumer's output tiles of a step, placed over the stage's KgT region
-// once the consumer has read it (loader 1, which refills that region, stores
-// them first)
-template <class E>
-struct __attribute__((aligned(16))) FwdScratch {
-  E s[16 * SC_SROW];  // state entering the chunk, [v][k]
-  E v[16 * SC_VROW];  // v_new, [v][t]
-};
-static_assert(sizeof(FwdScratch<bf16>) <= 128 * 64 * sizeof(bf16), "scratch must fit the KgT region");
-template <class E>
-__device__ __forceinline__ FwdScratch<E>& fwd_scratch(FwdStage<E>& st) {
-  return *reinterpret_cast<FwdScratch<E>*>(st.kg);
-}
-
-// Per-lane byte offsets of a loader's copies within a full chunk (the same for
-// every chunk of 64 events): part 0 the 16 W-row copies (from the chunk's first
-// event row), part 1 the 16 KgT copies and the 2 U^T copies (from the chunk's
-// tiles).  With them a full chunk's copy costs one address add.
-template <int PART>
-struct FwdCopyOffsets {
-  uint32_t o[PART == 0 ? 16 : 18];
-};
-template <class E, int PART>
-__device__ __forceinline__ FwdCopyOffsets<PART> fwd_copy_offsets(int H, int h, int lane) {
-  FwdCopyOffsets<PART> f;
-  if constexpr (PART == 0) {
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const int t = 4 * i + (lane >> 4), col = (lane & 15) ^ (t & 15);
-      f.o[i] = (uint32_t)(((t * H + h) * D + 8 * col) * sizeof(E));
-    }
-  } else {
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const int k = 8 * i + (lane >> 3), col = (lane & 7) ^ ((k >> 1) & 7);
-      f.o[i] = (uint32_t)((k * CH + 8 * col) * sizeof(E));
-    }
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int v = 8 * i + (lane >> 3), col = (lane & 7) ^ ((v >> 1) & 7);
-      f.o[16 + i] = (uint32_t)((v * CH + 8 * col) * sizeof(E));
-    }
-  }
-  return f;
-}
-
-// Issue the asynchronous copies of chunk c into stage S, in two parts: part 0
-// (loader 0) the -W rows and G_last, 17 copies; part 1 (loader 1) KgT and the
-// U^T slice, 18 copies.  Nothing here waits on memory: the chunk table is read
-// with scalar loads and even the gate value travels by copy (a vector load
-// whose result were used here would make this wave wait for every copy issued
-// before it).  A tail chunk re-reads its last W row for the rows past its
-// length (zeroed by fwd_fix_tail).
-constexpr int FWD_PART_COPIES[2] = {17, 18};
-template <class E, int PART>
-__device__ __forceinline__ void fwd_issue(FwdStage<E>& S, const int32_t* __restrict__ chunks, int c, int H, int h,
-                                          int v0, int lane, const FwdCopyOffsets<PART>& f,
-                                          const E* __restrict__ W, const E* __restrict__ UT,
-                                          const E* __restrict__ KgT, const float* __restrict__ gc) {
-  const ChunkInfo ci = chunk_info(chunks, c);
-  const size_t cb = (size_t)c * H + h;
-  if constexpr (PART == 0) {
-    if (ci.len == CH) {
-      const char* base = reinterpret_cast<const char*>(W + (size_t)ci.start * H * D);
-#pragma unroll
-      for (int i = 0; i < 16; ++i) dma16(base + f.o[i], S.w + 512 * i);
-    } else {
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const int t = 4 * i + (lane >> 4), col = (lane & 15) ^ (t & 15);
-        const int tt = min(t, ci.len - 1);
-        dma16(W + ((size_t)(ci.start + tt) * H + h) * D + 8 * col, S.w + 512 * i);
-      }
-    }
-    if (lane == 0)  // one lane: a dword copy writes 4 bytes per active lane
-      __builtin_amdgcn_global_load_lds(gc + (size_t)(ci.start + ci.len - 1) * H + h, (lds_void_ptr)&S.glast, 4, 0,
-                                       0);
-  } else {
-    const char* kg = reinterpret_cast<const char*>(KgT + cb * (D * CH));
-#pragma unroll
-    for (int i = 0; i < 16; ++i) dma16(kg + f.o[i], S.kg + 512 * i);
-    const char* ut = reinterpret_cast<const char*>(UT + cb * (D * CH) + v0 * CH);
-#pragma unroll
-    for (int i = 0; i < 2; ++i) dma16(ut + f.o[16 + i], S.ut + 512 * i);
-  }
-}
-
-// After the copies of chunk c have landed: zero the W rows past its length.
-template <class E>
-__device__ __forceinline__ void fwd_fix_tail(FwdStage<E>& S, const int32_t* __restrict__ chunks, int c, int lane) {
-  const int len = chunk_info(chunks, c).len;
-  if (len < CH) {
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const int t = 4 * i + (lane >> 4);
-      if (t >= len) st8(S.w + t * 128 + 8 * (lane & 15), zero8v<E>());
-    }
-  }
-}
-
-// global stores of one copy-out (4 of h^T, 2 of v_new^T)
-constexpr int FWD_OUT_STORES = 6;
-
-// scratch of one step -> hT [v0..v0+15][k], vnT [v0..v0+15][t]; NaN instead once
-// a hand-off wait has given up (the scratch may then hold another step's values)
-template <class E>
-__device__ __forceinline__ void fwd_copy_out(const FwdScratch<E>& sc, int c, int H, int h, int v0, int lane,
-                                             bool poison, E* __restrict__ hT, E* __restrict__ vnT) {
-  typedef typename Vec<E>::x8 X8;
-  const size_t cb = (size_t)c * H + h;
-  const X8 nan8 = to8<E>(f32x8{NAN, NAN, NAN, NAN, NAN, NAN, NAN, NAN});
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int seg = 64 * i + lane, v = seg >> 4, ks = seg & 15;
-    const X8 x = ld8(sc.s + v * SC_SROW + 8 * ks);
-    st8(hT + cb * (D * D) + (v0 + v) * D + 8 * ks, poison ? nan8 : x);
-  }
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const int seg = 64 * i + lane, v = seg >> 3, ts = seg & 7;
-    const X8 x = ld8(sc.v + v * SC_VROW + 8 * ts);
-    st8(vnT + cb * (D * CH) + (v0 + v) * CH + 8 * ts, poison ? nan8 : x);
-  }
-}
-
-// Loader PART of the forward scan, iteration x: publish chunk x-2 as soon as
-// this loader's part of it has landed, then, once the consumer is done with
-// chunk x-4, refill that chunk's stage (x % 4) with this loader's part of
-// chunk x (loader 1 first stores chunk x-4's outputs from the stage's KgT
-// region).  Loads and stores retire in issue order (one counter on gfx9), so a
-// loader waits for chunk x-2 by letting exactly the operations it issued after
-// that part stay in flight: its part of chunk x-1 and, for loader 1, the
-// copy-out before it.
-template <class E, int PART>
-__device__ __forceinline__ void fwd_loader(FwdStage<E>* stage, int* flags, const int32_t* __restrict__ chunks,
-                                           int c_begin, int n, int H, int h, int v0, int lane,
-                                           const E* __restrict__ W, const E* __restrict__ UT,
-                                           const E* __restrict__ KgT, const float* __restrict__ gc,
-                                           E* __restrict__ hT, E* __restrict__ vnT) {
-  const FwdCopyOffsets<PART> offs = fwd_copy_offsets<E, PART>(H, h, lane);
-  // Once a wait gives up, the rest run without waiting, and flags[3] tells the
-  // consumer, which turns its state (and so every later output) to NaN: stages
-  // refilled without the wait may be overwritten while it reads them.
-  bool ok = true;
-  for (int x = 0; x < n + SC_STAGES; ++x) {
-    const int y = x - 2;
-    if (y >= 0 && y < n) {
-      const int parts = x - 1 < n;
-      if constexpr (PART == 0) {
-        wait_vmem_parts<FWD_PART_COPIES[0], FWD_OUT_STORES>(parts, 0);
-        fwd_fix_tail(stage[y & (SC_STAGES - 1)], chunks, c_begin + y, lane);
-      } else {
-        wait_vmem_parts<FWD_PART_COPIES[1], FWD_OUT_STORES>(parts, x - 5 >= 0 && x - 5 < n);
-      }
-      lds_flag_publish(&flags[PART], y + 1);
-    }
-    if (x >= SC_STAGES) {
-      if (ok) {
-        ok = lds_flag_wait_ge<true>(&flags[2], x - SC_STAGES + 1);
-        if (!ok) {  // published (and complete in LDS) before this wave refills any stage
-          lds_flag_publish(&flags[3], 1);
-          asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        }
-      }
-      if (PART == 1 && x - SC_STAGES < n)
-        fwd_copy_out(fwd_scratch(stage[x & (SC_STAGES - 1)]), c_begin + x - SC_STAGES, H, h, v0, lane,
-                     lds_flag_read(&flags[3]) != 0, hT, vnT);
-    }
-    if (x < n) fwd_issue<E, PART>(stage[x & (SC_STAGES - 1)], chunks, c_begin + x, H, h, v0, lane, offs, W, UT, KgT, gc);
-  }
-}
-
-template <class E>
-__global__ __launch_bounds__(SC_THREADS) void fwd_scan_kernel(
-    const E* __restrict__ W, const E* __restrict__ UT, const E* __restrict__ KgT,
-    const float* __restrict__ gc, const int32_t* __restrict__ chunks, const int32_t* __restrict__ doc_chunk,
-    int H, const float* __restrict__ vscale, const float* __restrict__ init_state, float* __restrict__ final_state,
-    E* __restrict__ hT, E* __restrict__ vnT) {
+__global__ __launch_bounds__(SCAN_THREADS, 2) void fwd_scan_kernel(
+    // without __restrict__ where loads are requested ahead: the barriers then pin their place
+    const E* W, const E* UT, const E* KgT, const float* gc, const int32_t* chunks,
+    const int32_t* __restrict__ doc_chunk, int H, const float* __restrict__ vscale,
+    const float* __restrict__ init_state, float* __restrict__ final_state, E* hT, E* vnT) {
   typedef typename Vec<E>::x8 X8;
   typedef typename Vec<E>::x4 X4;
   // blockIdx.x = slice * H + h: the slices of one head land on one XCD when H % 8 == 0
   const int h = blockIdx.x % H, slice = blockIdx.x / H, d = blockIdx.y;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r = lane & 15, q4 = lane >> 4;
   const int v0 = 16 * slice;
 
-  __shared__ FwdStage<E> stage[SC_STAGES];
-  // hand-off counts: [0], [1] chunks whose part from loader 0 / 1 has landed
-  // (and, for loader 0, whose tail rows are zeroed); [2] chunks the consumer
-  // has finished (operands read, outputs in the stage's scratch); [3] nonzero
-  // once a loader's wait for the consumer has given up
-  __shared__ __attribute__((aligned(16))) int flags[4];
-  if (threadIdx.x < 4) flags[threadIdx.x] = 0;
-  __syncthreads();
+  __shared__ __attribute__((aligned(16))) E Sx[16 * SCAN_SROW];  // the state's operand copy, [v][perm32(k)]
+  __shared__ __attribute__((aligned(16))) E Vx[16 * SCAN_VROW];  // v_new, [v][perm32(t)]
+  // -W rows of SCAN_DEPTH chunks, each wave's 16 rows its own
+  __shared__ __attribute__((aligned(16))) E W0[64 * D], W1[64 * D], W2[64 * D], W3[64 * D];
+  static_assert(SCAN_DEPTH == 4, "four rings, and the waits below");
 
-  const int c_begin = doc_chunk[d], n = doc_chunk[d + 1] - c_begin;
-  if (wave == 0) {
-    f32x4 S[8];  // S[m][i] = state[k = 16m + 4q4 + i][v = v0 + r]
+  const int c_begin = __builtin_amdgcn_readfirstlane(doc_chunk[d]);
+  const int n = __builtin_amdgcn_readfirstlane(doc_chunk[d + 1]) - c_begin;
+  const float vs = vscale ? *vscale : 1.f;  // the state is carried in the scale of V
+  f32x4 S[2];  // S[m][i] = state[k = 32 wave + 16 m + 4 q4 + i][v = v0 + r]
 #pragma unroll
-    for (int m = 0; m < 8; ++m) S[m] = zero4();
-    const float vs = vscale ? *vscale : 1.f;  // the state is carried in the scale of V
-    if (init_state) {
-      const float* s0 = init_state + ((size_t)d * H + h) * D * D;
+  for (int m = 0; m < 2; ++m) S[m] = zero4();
+  if (init_state) {
+    const float* s0 = init_state + ((size_t)d * H + h) * D * D;
 #pragma unroll
-      for (int m = 0; m < 8; ++m)
+    for (int m = 0; m < 2; ++m)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) S[m][i] = s0[(16 * m + 4 * q4 + i) * D + v0 + r] * vs;
+      for (int i = 0; i < 4; ++i) S[m][i] = s0[(32 * wave + 16 * m + 4 * q4 + i) * D + v0 + r] * vs;
+  }
+  if (n > 0) {
+    ScanTable tab(chunks, gc, W, c_begin, 1, n, H, h, lane);
+    const size_t cb = (size_t)c_begin * H + h;
+    const int64_t tile = (int64_t)H * D * CH * 2;  // bytes from one chunk's [D][64] tile to the next chunk's
+    ScanBlocks<false> kb(KgT + cb * (D * CH), tile, n), ub(UT + cb * (D * CH) + v0 * CH, tile, n);
+    ScanBlocks<false> vb(vnT + cb * (D * CH) + v0 * CH, tile, n), hb(hT + cb * (D * D) + v0 * D, 2 * tile, n);
+    // per-lane parts of the addresses, the same for every chunk (bytes of global
+    // memory; elements of LDS)
+    const int q = (lane >> 2) & 3, p = lane & 3, from = tile_source(lane);
+    int w_off[4], w_in[4];  // -W rows 16 wave + 4 i + q4, column r ^ row; fragment j: row 16 wave + r, column 4 q4 + j
+#pragma unroll
+    for (int i = 0; i < 4; ++i) w_off[i] = (16 * wave + 4 * i + q4) * H * D * 2 + 16 * (r ^ (4 * i + q4));
+    E* const ring[SCAN_DEPTH] = {W0, W1, W2, W3};
+#pragma unroll
+    for (int j = 0; j < 4; ++j) w_in[j] = (16 * wave + r) * D + 8 * ((4 * q4 + j) ^ r);
+    const int k_off = 4096 * wave + 16 * lane;                    // fragments (wave, m, b) of KgT
+    const int u_off = (4 * q4 + q) * CH * 2 + 32 * wave + 8 * p;  // U^T row 4 q4 + q, t = 16 wave + 4 p ..
+    const int s_own = r * SCAN_SROW + 32 * wave + 8 * q4, s_in = r * SCAN_SROW + 32 * q4;
+    const int v_own = r * SCAN_VROW + 32 * (wave >> 1) + 8 * q4 + 4 * (wave & 1), v_in = r * SCAN_VROW + 8 * q4;
+    // the outputs as rows: h^T row 4 wave + q4, k = 8 r .. 8 r + 7 (two runs of four in
+    // perm32 order), v_new^T row 4 wave + q4, t = 4 r .. 4 r + 3
+    const int s_row = (4 * wave + q4) * SCAN_SROW, s_lo = s_row + perm32(8 * r), s_hi = s_row + perm32(8 * r + 4);
+    const int v_row = (4 * wave + q4) * SCAN_VROW + perm32(4 * r);
+    const int h_off = 1024 * wave + 16 * lane, vn_off = 512 * wave + 8 * lane;
+    X8 fk[SCAN_DEPTH][2][2];
+    X4 fu[SCAN_DEPTH], u;
+    X8 w[4];
+    float gl[SCAN_DEPTH];
+    // l: the step's place after the table's and the blocks' first
+    auto issue_w = [&](int slot, int l) __attribute__((always_inline)) {
+      const __amdgpu_buffer_rsrc_t wr = tab.rows(l), ur = ub.buffer();
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(wr, (lds_void_ptr)(ring[slot] + (16 * wave + 4 * i) * D), 16,
+                                                 w_off[i], 0, 0, 0);
+      fu[slot] = buf_ld8<X4>(ur, u_off, ub.offset(l));
+      gl[slot] = tab.glast(l);
+    };
+    auto issue_k = [&](int slot, int l) __attribute__((always_inline)) {
+      const __amdgpu_buffer_rsrc_t kr = kb.buffer();
+#pragma unroll
+      for (int m = 0; m < 2; ++m)
+#pragma unroll
+        for (int b = 0; b < 2; ++b) fk[slot][m][b] = buf_ld16<X8>(kr, k_off + 2048 * m + 1024 * b, kb.offset(l));
+    };
+    st8(Sx + s_own, pack_permv<E>(S[0], S[1]));
+#pragma unroll
+    for (int x = 0; x < SCAN_DEPTH; ++x) {
+      issue_w(x, x);
+      issue_k(x, x);
+      __builtin_amdgcn_sched_barrier(0);  // in this order: the waits count on it
     }
-    // per-lane parts of the swizzled LDS addresses (bytes); the row parts are
-    // compile-time offsets of each read
-    int wofs[4], kofs[2], uofs[4];
+    // -W of the next step, once at most `flight` operations are in flight
+    auto take_w = [&](auto flight, int slot) __attribute__((always_inline)) {
+      wait_vmem_le<decltype(flight)::value>();
+      asm volatile("" ::: "memory");
 #pragma unroll
-    for (int j = 0; j < 4; ++j) wofs[j] = 2 * (r * 128 + 8 * ((4 * j + q4) ^ r));
+      for (int j = 0; j < 4; ++j) w[j] = ld8(ring[slot] + w_in[j]);
+    };
+    float g_now = __expf(gl[0]);
+    u = tile_exchange(fu[0], from);
+    take_w(Int<3 * FWD_LOAD_OPS>(), 0);
+    ub.advance();
+    kb.advance();
+    lds_barrier();
+    // one step: its -W, U and decay are in w, u and g_now; place: its place in the round;
+    // more: not one of the last steps, whose requests would all lie past the end; flight:
+    // operations surely issued after the next step's -W
+    auto step = [&](auto place, auto more, auto flight) __attribute__((always_inline)) {
+      constexpr int s = decltype(place)::value;
+      // v_new = U + (-W) S
+      X8 sx[4];
 #pragma unroll
-    for (int j = 0; j < 2; ++j) kofs[j] = 2 * (r * 64 + 8 * ((4 * j + q4) ^ ((r >> 1) & 7)));
+      for (int j = 0; j < 4; ++j) sx[j] = ld8(Sx + s_in + 8 * j);
+      const X8 h_out = cat(ld4(Sx + s_lo), ld4(Sx + s_hi));
+      f32x4 acc = cvtf4(u);
 #pragma unroll
-    for (int i4 = 0; i4 < 4; ++i4) uofs[i4] = 2 * (r * 64 + 8 * ((2 * i4 + (q4 >> 1)) ^ ((r >> 1) & 7)) + 4 * (q4 & 1));
-    const int sofs = 2 * (r * SC_SROW + 4 * q4), vofs = 2 * (r * SC_VROW + 4 * q4);
-    int seen = 0;       // both loaders' counts are at least this (last read)
-    bool ok = true;     // every hand-off wait succeeded
-    int poisoned = 0;   // flags[3] as last read
-    for (int tau = 0; tau < n; ++tau) {
-      if (ok && seen <= tau) ok = scan_wait_ready(flags, tau + 1, seen);
-      if (poisoned) ok = false;
-      if (!ok) {  // a broken hand-off: make every later output NaN
-        // (the empty asm keeps this a branch: as selects it cost 32 VALU operations a step)
-        asm volatile("");
+      for (int j = 0; j < 4; ++j) acc = mfma(w[j], sx[j], acc);
+      buf_st16(hb.buffer(), h_off + hb.offset(s), h_out);
 #pragma unroll
-        for (int m = 0; m < 8; ++m) S[m] = f32x4{NAN, NAN, NAN, NAN};
-      }
-      char* base = reinterpret_cast<char*>(&stage[tau & (SC_STAGES - 1)]);
-      const char* wb = base + offsetof(FwdStage<E>, w);
-      const char* kb = base + offsetof(FwdStage<E>, kg);
-      const char* ub = base + offsetof(FwdStage<E>, ut);
-      // every operand read is issued ahead of the MFMAs that use them (the W
-      // fragments first); the scheduling barriers keep the compiler from
-      // interleaving them one by one
-      X8 fw[4][4], fk[8][2];
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-#pragma unroll
-        for (int i4 = 0; i4 < 4; ++i4) fw[i4][j] = *reinterpret_cast<const X8*>(wb + wofs[j] + 4096 * i4);
-      f32x4 vn[4];
-#pragma unroll
-      for (int i4 = 0; i4 < 4; ++i4) vn[i4] = cvtf4(*reinterpret_cast<const X4*>(ub + uofs[i4]));
-      const float glast = reinterpret_cast<const FwdStage<E>*>(base)->glast;
-#pragma unroll
-      for (int j = 0; j < 2; ++j)
-#pragma unroll
-        for (int m = 0; m < 8; ++m) fk[m][j] = *reinterpret_cast<const X8*>(kb + kofs[j] + 2048 * m);
-      const int2 pre = lds_flag_read2(flags);  // for the next step, read while this one computes
-      poisoned = lds_flag_read(&flags[3]);
-      __builtin_amdgcn_sched_barrier(0);
-      X4 sh[8];
-#pragma unroll
-      for (int m = 0; m < 8; ++m) sh[m] = to4<E>(S[m]);
-      // v_new = U + (-W) S; the state's decay runs beside it
-      const float gC = __expf(glast);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const X8 hb = cat(sh[2 * j], sh[2 * j + 1]);
-#pragma unroll
-        for (int i4 = 0; i4 < 4; ++i4) vn[i4] = mfma(fw[i4][j], hb, vn[i4]);
-#pragma unroll
-        for (int m = 2 * j; m < 2 * j + 2; ++m) S[m] *= gC;
-      }
-      __builtin_amdgcn_sched_barrier(0);
-      // the KgT fragments have been read (a wave's LDS operations complete in
-      // order): the KgT region now takes this step's outputs
-      char* sb = base + offsetof(FwdStage<E>, kg);
-#pragma unroll
-      for (int m = 0; m < 8; ++m) *reinterpret_cast<X4*>(sb + sofs + 32 * m) = sh[m];
+      for (int m = 0; m < 2; ++m) S[m] *= g_now;
+      *reinterpret_cast<X4*>(Vx + v_own) = to4<E>(acc);
+      lds_barrier();
       // S <- exp(G_last) S + (K exp(G_last - G))^T v_new
+      const X8 b0 = ld8(Vx + v_in), b1 = ld8(Vx + v_in + 32);
+      const X4 v_out = ld4(Vx + v_row);
+      const int next = (s + 1) % SCAN_DEPTH;
+      g_now = __expf(gl[next]);
+      take_w(flight, next);
+      u = tile_exchange(fu[next], from);
 #pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        const X8 vb = pack_permv<E>(vn[2 * j], vn[2 * j + 1]);
+      for (int m = 0; m < 2; ++m) S[m] = mfma(fk[s][m][0], b0, S[m]);
 #pragma unroll
-        for (int m = 0; m < 8; ++m) S[m] = mfma(fk[m][j], vb, S[m]);
+      for (int m = 0; m < 2; ++m) S[m] = mfma(fk[s][m][1], b1, S[m]);
+      if constexpr (decltype(more)::value) {
+        issue_w(s, s);
+        issue_k(s, s);
       }
-      char* vbp = sb + sizeof(FwdScratch<E>::s);
-#pragma unroll
-      for (int i4 = 0; i4 < 4; ++i4) *reinterpret_cast<X4*>(vbp + vofs + 32 * i4) = to4<E>(vn[i4]);
-      lds_flag_publish(&flags[2], tau + 1);
-      seen = max(seen, min(__builtin_amdgcn_readfirstlane(pre.x), __builtin_amdgcn_readfirstlane(pre.y)));
+      buf_st8(vb.buffer(), vn_off, vb.offset(s), v_out);
+      st8(Sx + s_own, pack_permv<E>(S[0], S[1]));
+      lds_barrier();
+    };
+    // SCAN_DEPTH steps a round, so that the operand ring's registers are named by constants
+    auto round = [&](int tau, auto flight) __attribute__((always_inline)) {
+      tab.advance(tau + SCAN_DEPTH);
+      step(Int<0>(), Int<1>(), flight);
+      step(Int<1>(), Int<1>(), flight);
+      step(Int<2>(), Int<1>(), flight);
+      step(Int<3>(), Int<1>(), flight);
+      ub.advance();
+      kb.advance();
+      vb.advance();
+      hb.advance();
+    };
+    int tau = 0;
+    if (n >= SCAN_DEPTH) {
+      // its first step's next -W has two more slots' loads after it and this step's store
+      round(0, Int<2 * FWD_LOAD_OPS + 1>());
+      for (tau = SCAN_DEPTH; tau + SCAN_DEPTH <= n; tau += SCAN_DEPTH) round(tau, Int<2 * FWD_STEP_OPS + 1>());
     }
-    if (final_state) {
-      float* sf = final_state + ((size_t)d * H + h) * D * D;
-      const float inv = 1.f / vs;  // exact: vs is a power of two
+    // the last steps issue their two stores only (and n < SCAN_DEPTH never issued more than the first loads)
+    if (tau < n) step(Int<0>(), Int<0>(), Int<2 * FWD_LOAD_OPS + 1>());
+    if (tau + 1 < n) step(Int<1>(), Int<0>(), Int<FWD_LOAD_OPS + 3>());
+    if (tau + 2 < n) step(Int<2>(), Int<0>(), Int<5>());
+  }
+  if (final_state) {
+    float* sf = final_state + ((size_t)d * H + h) * D * D;
+    const float inv = 1.f / vs;  // exact: vs is a power of two
 #pragma unroll
-      for (int m = 0; m < 8; ++m)
+    for (int m = 0; m < 2; ++m)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) sf[(16 * m + 4 * q4 + i) * D + v0 + r] = S[m][i] * inv;
-    }
-  } else {
-    // The loader's part is a template argument, so its copy offsets stay in
-    // registers (indexed by a run-time part they went to scratch memory, and
-    // reloading them waited for every copy in flight).
-    if (wave == 1)
-      fwd_loader<E, 0>(stage, flags, chunks, c_begin, n, H, h, v0, lane, W, UT, KgT, gc, hT, vnT);
-    else
-      fwd_loader<E, 1>(stage, flags, chunks, c_begin, n, H, h, v0, lane, W, UT, KgT, gc, hT, vnT);
+      for (int i = 0; i < 4; ++i) sf[(32 * wave + 16 * m + 4 * q4 + i) * D + v0 + r] = S[m][i] * inv;
   }
 }
 
@@ -895,7 +762,7 @@ static hipError_t launch_fwd_t(const FwdArgs& a, float* vscale, int vs_target, h
   }
   {
     TimedLaunch tl(K_FWD_SCAN, ss);
-    hipLaunchKernelGGL(fwd_scan_kernel<E>, grid_s, dim3(SC_THREADS), 0, ss, ws[F_W], ws[F_UT], ws[F_KGT], gcum,
+    hipLaunchKernelGGL(fwd_scan_kernel<E>, grid_s, dim3(SCAN_THREADS), 0, ss, ws[F_W], ws[F_UT], ws[F_KGT], gcum,
                        a.chunks, a.doc_chunk, a.H, vscale, a.initial_state, a.final_state, ws[F_HT], ws[F_VNT]);
   }
   if (a.scan_stream)

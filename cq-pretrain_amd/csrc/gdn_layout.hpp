@@ -18,7 +18,9 @@
 // buffers ([8][rows][16]: slice s holds values 16 s .. 16 s + 15 of every row)
 // are written by the state scans, whose workgroups each own one 16-wide value
 // slice: a scan step stores one contiguous block, and a reader's MFMA fragment
-// (8 consecutive values of one row) is one contiguous 16-byte load.
+// (8 consecutive values of one row) is one contiguous 16-byte load.  A scan's own
+// operands are stored fragment by fragment, the 16 bytes of each lane in lane
+// order, so that a fragment is one contiguous kilobyte.
 #pragma once
 #include <stddef.h>
 #include <stdint.h>
@@ -31,7 +33,7 @@ enum FwdBuf {
   F_TM,      // bf16 [NC][H][64][64]  T = (I + A)^-1, row-major (t, s)
   F_W,       // bf16 [T][H][D]   -W, W = T (beta*exp(G)*K), rows (t, k), perm32 column order
   F_UT,      // bf16 [NC][H][D][64]   U = T (beta*V) transposed (v, t)
-  F_KGT,     // bf16 [NC][H][D][64]   (K * exp(G_last - G)) transposed (k, t), perm32 columns
+  F_KGT,     // bf16 [NC][H][D][64]   (K * exp(G_last - G)) transposed, in the forward scan's fragment order
   F_HT,      // bf16 [NC][H][D][D]    state entering the chunk, (v, k)
   F_VNT,     // bf16 [NC][H][D][64]   v_new transposed (v, t)
   F_VSC,     // f32  [1 + 1024]       power-of-two scale s_v of V and block partials (fp16 operands)
@@ -43,8 +45,8 @@ enum BwdBuf {
   B_XT,        // bf16 [NC][H][D][D]   X = scale*(gam*Qn)^T dO, (v, k)
   B_DH,        // bf16 [NC][H][8][D][16]  gradient of the state leaving the chunk, value-slice-major (s, k, v%16)
   B_DVN,       // bf16 [NC][H][8][64][16] d v_new, value-slice-major (s, t, v%16)
-  B_KNP,       // bf16 [T][H][D]       exp(G_last - G_t) Kn_t in perm32 column order (reverse scan operand), by bwd_local
-  B_WT,        // bf16 [NC][H][D][64]  -W transposed (k, t), perm32 column order (reverse scan operand), by bwd_local
+  B_KNP,       // bf16 [NC][H][64][D]  exp(G_last - G_t) Kn_t in the reverse scan's fragment order, by bwd_local
+  B_WT,        // bf16 [NC][H][D][64]  -W transposed in the reverse scan's fragment order, by bwd_local
   B_SYNC,      // i32  [NC][H] + 64     per (chunk, head): reverse-scan value slices whose dS / dVn are stored,
                //                       then at [NC][H] the count of resident reverse-scan workgroups
                //                       (bwd_dkw beside the scan; zeroed by bwd_local)
@@ -79,7 +81,7 @@ inline void bwd_sizes(int64_t T, int64_t H, int64_t NC, size_t* s) {
   s[B_XT] = chunk * 128 * 128 * 2;
   s[B_DH] = chunk * 128 * 128 * 2;
   s[B_DVN] = chunk * 64 * 128 * 2;
-  s[B_KNP] = ev * 128 * 2;
+  s[B_KNP] = chunk * 64 * 128 * 2;
   s[B_WT] = chunk * 128 * 64 * 2;
   s[B_SYNC] = (chunk + 64) * 4;
   s[B_DSC] = (1 + kVscaleBlocks) * 4;
