@@ -468,6 +468,12 @@ __global__ __launch_bounds__(SCAN_THREADS, 2) void bwd_scan_kernel(
 // reads accordingly).
 // The l2norm backward of dq runs on the phase-2 registers (per-wave row dots in
 // LDS), so no fp32 staging tile is needed and dQ's registers carry the dK partial.
+// h is read by whole row pieces and turned in LDS (columns_from_rows), and dq, dk and dv
+// leave as whole rows, dq through the dO rows' place before the dVn copy, dk and dv from
+// the K and V rows' places, whose values only their lane still reads: column gathers and
+// 8-byte stores from lanes on 16 different rows keep the vector memory unit 3 and 2.5
+// times as long.  H = 16, 144 chunks / 520 chunks of 15 documents / 36 chunks: 127.5 ->
+// 122.4 / 420 -> 402 / 42.5 -> 40.8 us (the stores alone gave 3, the gathers 1.5).
 // Barriers order LDS only (s_waitcnt lgkmcnt(0); s_barrier): global stores stay
 // in flight across them, and the one barrier that needs the dVn tile's copies
 // waits for vector memory explicitly.
@@ -535,12 +541,10 @@ __global__ __launch_bounds__(256, 2) void bwd_dkw_kernel(
   // way), the v_new^T rows and the Q, K, dO rows; the gathers' lane exchange
   // comes last.  The q norm is formed from the Q rows (row_rnorm).
   {
-    Col8 gh[2][4];
-#pragma unroll
-    for (int mm = 0; mm < 2; ++mm)
-#pragma unroll
-      for (int kb = 0; kb < 4; ++kb) gh[mm][kb] = col8_load(ht, D, 32 * kb, 16 * (2 * wave + mm));
     const int t = tid >> 2, p = tid & 3;
+    X8 gh[8];  // h^T row v = 16 i + lane / 4, piece p of the wave's columns k = 32 wave ..
+#pragma unroll
+    for (int i = 0; i < 8; ++i) gh[i] = row_piece(ht, D, 16 * i + (lane >> 2), 32 * wave);
     const bool in = t < ci.len;
     const int tc = clamp_row(t, ci.len);
     const size_t ev = (size_t)(ci.start + tc) * H + h, row = ev * D;
@@ -583,10 +587,14 @@ __global__ __launch_bounds__(256, 2) void bwd_dkw_kernel(
       st8(Ks + t * LDK + col, keep_if(in, scaled8<E>(xk[j], rkv)));
       st8(dOs + t * LDK + col, keep_if(in, xo[j]));
     }
+    // through dPm's region, whose first use is after the barrier
 #pragma unroll
-    for (int mm = 0; mm < 2; ++mm)
-#pragma unroll
-      for (int kb = 0; kb < 4; ++kb) bh[mm][kb] = col8_combine_v<E>(gh[mm][kb]);
+    for (int kb = 0; kb < 4; ++kb) {
+      X8 y[2];
+      columns_from_rows(dPm + 1024 * wave, gh[2 * kb], gh[2 * kb + 1], y);
+      bh[0][kb] = y[0];
+      bh[1][kb] = y[1];
+    }
   }
   lds_barrier();
   const float glast = Gs[ci.len - 1];
@@ -741,7 +749,10 @@ __global__ __launch_bounds__(256, 2) void bwd_dkw_kernel(
   // dq = rq (dQ - q (q . dQ)): each lane stores 4 consecutive k of row t = 16 n + r
   const int rowb = H * D * 2;  // bytes per event row
   {
+  // dq's rows over the dO rows (256-byte rows, 16-byte columns XORed with t % 16), then
+  // whole rows to memory: a store whose lanes are rows costs 2.5 times the whole rows' time
   const __amdgpu_buffer_rsrc_t dq_rs = chunk_rows_rsrc(dq, ci.start, ci.len, H, h);
+  E* dqs = dOs;
 #pragma unroll
   for (int n = 0; n < 4; ++n) {
     const int t = 16 * n + r;
@@ -752,9 +763,20 @@ __global__ __launch_bounds__(256, 2) void bwd_dkw_kernel(
     for (int mm = 0; mm < 2; ++mm) {
       const int k0 = 16 * (2 * wave + mm) + 4 * q4;
       const f32x4 x = normalize ? (dQ[mm][n] - qrow[n][mm] * dot) * rs : dQ[mm][n];
-      buf_st4<E>(dq_rs, r * rowb + k0 * 2, 16 * n * rowb, F16 ? x * inv_dv : x);  // row t, columns k0 .. k0 + 3
+      st4(dqs + t * D + 8 * ((k0 >> 3) ^ r) + (k0 & 4), F16 ? x * inv_dv : x);  // row t, columns k0 .. k0 + 3
     }
   }
+  lds_barrier();
+  X8 rows[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) rows[i] = ld8(dqs + 512 * (4 * i + wave) + 8 * lane);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int t = 16 * i + 4 * wave + q4;
+    buf_st16(dq_rs, t * rowb + 16 * (r ^ (t & 15)), rows[i]);
+  }
+  // this wave's pieces are read: the dVn copies below take exactly their places
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   }
   // the dVn tile, copied global -> LDS while phase 3 runs (after the dq stores, which retire first)
   {
@@ -1022,7 +1044,6 @@ __global__ __launch_bounds__(256, 2) void bwd_dkw_kernel(
   wait_vmem_all();
   // ---- wy phase 4b: dv = beta (T^T dVn) ----
   {
-    const __amdgpu_buffer_rsrc_t dv_rs = chunk_rows_rsrc(dv, ci.start, ci.len, H, h);
     float colB[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int mm = 0; mm < 2; ++mm) {
@@ -1042,8 +1063,8 @@ __global__ __launch_bounds__(256, 2) void bwd_dkw_kernel(
         const int s = 16 * n + r;
         const f32x4 vv = cvtf4(ld4(Vs + s * LDK + 16 * m + 4 * q4));
         colB[n] += acc[n][0] * vv[0] + acc[n][1] * vv[1] + acc[n][2] * vv[2] + acc[n][3] * vv[3];
-        buf_st4<E>(dv_rs, r * rowb + (16 * m + 4 * q4) * 2, 16 * n * rowb,
-                   acc[n] * (F16 ? Bs[s] * inv_d : Bs[s]));  // row s
+        // over the V values that only this lane reads from here on
+        st4(Vs + s * LDK + 16 * m + 4 * q4, acc[n] * (F16 ? Bs[s] * inv_d : Bs[s]));
       }
     }
 #pragma unroll
@@ -1111,7 +1132,12 @@ __global__ __launch_bounds__(256, 2) void bwd_dkw_kernel(
   lds_barrier();
 
   // ---- wy phase 5: l2norm backward of dk; dg (reverse cumsum of the chunk's dG); dbeta ----
+  // dv and dk leave as whole rows, dv from the V rows' place, dk from the K rows'
   const __amdgpu_buffer_rsrc_t dk_rs = chunk_rows_rsrc(dk, ci.start, ci.len, H, h);
+  const __amdgpu_buffer_rsrc_t dv_rs = chunk_rows_rsrc(dv, ci.start, ci.len, H, h);
+  const int row_l = (tid >> 2) * LDK + 8 * (tid & 3), row_g = (tid >> 2) * rowb + 16 * (tid & 3);
+#pragma unroll
+  for (int j = 0; j < 4; ++j) buf_st16(dv_rs, row_g + 64 * j, ld8(Vs + row_l + 32 * j));
 #pragma unroll
   for (int n = 0; n < 4; ++n) {
     const int t = 16 * n + r;
@@ -1121,9 +1147,12 @@ __global__ __launch_bounds__(256, 2) void bwd_dkw_kernel(
     for (int mm = 0; mm < 2; ++mm) {
       const int m = 2 * wave + mm;
       const f32x4 out = normalize ? (dkr[mm][n] - krow[n][mm] * dot) * rsn[n] : dkr[mm][n];
-      buf_st4<E>(dk_rs, r * rowb + (16 * m + 4 * q4) * 2, 16 * n * rowb, F16 ? out * inv_dv : out);  // row t
+      st4(Ks + t * LDK + 16 * m + 4 * q4, F16 ? out * inv_dv : out);
     }
   }
+  lds_barrier();
+#pragma unroll
+  for (int j = 0; j < 4; ++j) buf_st16(dk_rs, row_g + 64 * j, ld8(Ks + row_l + 32 * j));
   if (tid < 64) {
     const int t = tid;
     const bool in = t < ci.len;

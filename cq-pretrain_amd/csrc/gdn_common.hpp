@@ -299,6 +299,38 @@ __device__ __forceinline__ typename Vec<E>::x8 col8_combine_v(const Col8& g) {
   return __builtin_bit_cast(typename Vec<E>::x8, col8_combine(g));
 }
 
+// MFMA fragments of the columns of a row-major matrix M in global memory, for a wave that
+// needs 32 columns c0 .. c0 + 31: the rows are read by quads (row_piece: lane l reads row
+// l / 4 of 16, 16-byte piece l % 4; 64 bytes of a row a quad, the rate of whole rows, where
+// dword gathers down the columns measured 3 times slower), and 32 rows at a time pass
+// through 2 KB of LDS of the wave's own: columns_from_rows takes rows 0 .. 15 (x0) and 16
+// .. 31 (x1) and returns for the two 16-column tiles the fragment ld8 would give of M^T:
+// lane (q4, r) gets M[8 q4 + e][16 m + r], e = 0..7.  The LDS rows' 16-byte columns are
+// XORed with (row / 2) % 4, so that the 4 rows x 32 bytes a lane group reads spread over
+// the banks.  A wave's LDS operations complete in order, so no barrier is needed.
+template <class T>  // bf16 or f16
+__device__ __forceinline__ typename Vec<T>::x8 row_piece(const T* M, size_t ld, int row, int c0) {
+  return ld8(M + row * ld + c0 + 8 * (threadIdx.x & 3));
+}
+template <class T>
+__device__ __forceinline__ void columns_from_rows(T* own, typename Vec<T>::x8 x0, typename Vec<T>::x8 x1,
+                                                  typename Vec<T>::x8 (&y)[2]) {
+  typedef __attribute__((address_space(3))) i16x4 lds_i16x4;
+  const int lane = threadIdx.x & 63, r = lane & 15, q4 = lane >> 4;
+  T* const w = own + (lane >> 2) * 32 + 8 * ((lane & 3) ^ ((lane >> 3) & 3));
+  st8(w, x0);
+  st8(w + 512, x1);
+  const T* const t = own + (8 * q4 + (r >> 2)) * 32 + 4 * (r & 1);  // rows 8 q4 + r / 4, then 4 further on
+  const int sw = (r >> 3) & 1;
+#pragma unroll
+  for (int m = 0; m < 2; ++m) {
+    const int c = 2 * m + ((r >> 1) & 1);
+    const i16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(t + 8 * (c ^ sw)));
+    const i16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(t + 128 + 8 * (c ^ (2 + sw))));
+    y[m] = __builtin_bit_cast(typename Vec<T>::x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+  }
+}
+
 // ---- workgroup synchronization for loader/consumer kernels ----------------
 // Barrier that orders LDS only: waits for this wave's LDS operations, then
 // s_barrier.  __syncthreads() also waits for every outstanding vector-memory
