@@ -370,7 +370,11 @@ __global__ __launch_bounds__(256, 3) void fwd_prep_kernel(
 //   -W    rows go to LDS by asynchronous copies of four 256-byte rows (16-byte columns
 //         XOR-swizzled by row), each wave its own 16 rows, and come back as fragments;
 //   U^T   is read by quads and exchanged between lanes (tile_exchange);
-//   h^T, v_new^T leave as whole rows, read back from the LDS copies.
+//   h^T, v_new^T leave as whole rows, read back from the LDS copies; h^T with the
+//   non-temporal hint: its 32 KB a chunk-head would push the operands of the chunks still
+//   to come, and then bwd_local's, out of the memory-side cache (a training step of 144
+//   chunks 477 -> 464 us, packed 1496 -> 1484, 36 chunks 140.1 -> 139.4; v_new^T as well
+//   slowed fwd_out by 3 us and gained nothing more on a step).
 // With fragments read straight from the row-major matrices the same kernel took 173 us.
 // Operands are requested SCAN_DEPTH steps ahead into registers (and four LDS rings);
 // 3, 5 or 6 steps measured the same.  No step computes an address (ScanBlocks, ScanTable)
@@ -499,7 +503,7 @@ __global__ __launch_bounds__(SCAN_THREADS, 2) void fwd_scan_kernel(
       f32x4 acc = cvtf4(u);
 #pragma unroll
       for (int j = 0; j < 4; ++j) acc = mfma(w[j], sx[j], acc);
-      buf_st16(hb.buffer(), h_off + hb.offset(s), h_out);
+      buf_st16<CPOL_NT>(hb.buffer(), h_off + hb.offset(s), h_out);
 #pragma unroll
       for (int m = 0; m < 2; ++m) S[m] *= g_now;
       *reinterpret_cast<X4*>(Vx + v_own) = to4<E>(acc);
