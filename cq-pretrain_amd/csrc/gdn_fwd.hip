@@ -66,16 +66,13 @@ __global__ __launch_bounds__(256, 3) void fwd_prep_kernel(
   // Every global load is issued first, before any store (a wait for a load
   // also waits for every store issued before it), so the kernel pays one memory
   // round trip: the gates (wave 0), this thread's pieces of its k row,
-  // and this wave's operand fragments of V for U = T (beta V), column gathers
-  // for value tiles 2 wave, 2 wave + 1 (rows past the chunk re-read its last
-  // row; their beta is zero).  Each phase waits only for what it reads: the
-  // gathers' lane exchange runs where U is formed, and the stores of the row
-  // phase go through buffer resources (rows past the chunk dropped by the range
+  // and the columns 32 wave .. of V for U = T (beta V) (rows past the chunk re-read
+  // its last row; their beta is zero).  Each phase waits only for what it reads, and
+  // the stores of the row phase go through buffer resources (rows past the chunk dropped by the range
   // check), so no store is conditional and the compiler can count what is in flight.
   // k is loaded non-temporally: nothing reads it again before the state scan,
   // whose operands (written here) then keep more of the memory-side cache.  q is
   // not read here: its l2 scale is formed by each kernel that reads q (row_rnorm).
-  // (V's column gathers share lines between lanes and stay ordinary loads.)
   const int t_r = tid >> 2, p_r = tid & 3;  // row phase: thread (t, p) owns columns 8p + 32j, j = 0..3
   const size_t row_r = ((size_t)(ci.start + clamp_row(t_r, ci.len)) * H + h) * D;
   float gv = 0.f, bv = 0.f;
@@ -85,16 +82,12 @@ __global__ __launch_bounds__(256, 3) void fwd_prep_kernel(
     bv = beta[ev];
   }
   typename Vec<I>::x8 lk[4];
-  Col8 vg[2][2];
+  typename Vec<I>::x8 vr[4], vg[2][2];  // V rows 16 i + lane / 4 by quads, then the fragments (tile nn, t block kb)
 #pragma unroll
   for (int j = 0; j < 4; ++j) lk[j] = ld8_nt(k + row_r + 32 * j + 8 * p_r);
-  {
-    const I* vb = v + ((size_t)ci.start * H + h) * D;
 #pragma unroll
-    for (int nn = 0; nn < 2; ++nn)
-#pragma unroll
-      for (int kb = 0; kb < 2; ++kb) vg[nn][kb] = col8_load_rows(vb, H * D, 32 * kb, 16 * (2 * wave + nn), ci.len);
-  }
+  for (int i = 0; i < 4; ++i)
+    vr[i] = row_piece(v + ((size_t)ci.start * H + h) * D, (size_t)H * D, clamp_row(16 * i + (lane >> 2), ci.len), 32 * wave);
   // the scale of V, while the loads above are in flight (stored for the kernels
   // after this one at the end, where the store holds up no wait for a load)
   float vs = 1.f;
@@ -158,6 +151,14 @@ __global__ __launch_bounds__(256, 3) void fwd_prep_kernel(
       }
       buf_stf(rk_rs, t * H * 4, 0, rs);
     }
+  }
+  // the V fragments, through the place of T (written after the solve)
+#pragma unroll
+  for (int kb = 0; kb < 2; ++kb) {
+    typename Vec<I>::x8 y[2];
+    columns_from_rows(reinterpret_cast<I*>(Ts) + 1024 * wave, vr[2 * kb], vr[2 * kb + 1], y);
+    vg[0][kb] = y[0];
+    vg[1][kb] = y[1];
   }
   __syncthreads();
 
@@ -293,8 +294,8 @@ __global__ __launch_bounds__(256, 3) void fwd_prep_kernel(
   // beta gam K is read transposed from its rows (ld8_tr); beta V comes from the
   // V fragments gathered at the start, scaled here.  (-W^T, the reverse scan's
   // operand, is formed by bwd_local.)
+  X4 uo[2][4], wo[2][4];
   {
-    // U^T rows v = 16 (2 wave + nn) + 4 q4 .., all t tiles
     X8 bvf[2][2];
 #pragma unroll
     for (int kb = 0; kb < 2; ++kb) {
@@ -302,9 +303,8 @@ __global__ __launch_bounds__(256, 3) void fwd_prep_kernel(
       const f32x4 b1 = *reinterpret_cast<const f32x4*>(Bs + 32 * kb + 8 * q4 + 4);
       const f32x8 bb = f32x8{b0[0], b0[1], b0[2], b0[3], b1[0], b1[1], b1[2], b1[3]} * vs;
 #pragma unroll
-      for (int nn = 0; nn < 2; ++nn) bvf[nn][kb] = to8<E>(cvtf8(col8_combine_v<I>(vg[nn][kb])) * bb);
+      for (int nn = 0; nn < 2; ++nn) bvf[nn][kb] = to8<E>(cvtf8(vg[nn][kb]) * bb);
     }
-    E* ut = UT + cb * (D * CH);
 #pragma unroll
     for (int tt = 0; tt < 4; ++tt) {
       X8 a[2];
@@ -316,10 +316,9 @@ __global__ __launch_bounds__(256, 3) void fwd_prep_kernel(
 #pragma unroll
         for (int kb = 0; kb < 2; ++kb)
           if (kb == 0 || tt >= 2) au = mfma(a[kb], bvf[nn][kb], au);  // T[t][s] = 0 for s > t
-        st4(ut + (16 * (2 * wave + nn) + r) * CH + 16 * tt + 4 * q4, au);
+        uo[nn][tt] = to4<E>(au);
       }
     }
-    const __amdgpu_buffer_rsrc_t w_rs = buf_rsrc(W + ((size_t)ci.start * H + h) * D, rows_bytes);
 #pragma unroll
     for (int mm = 0; mm < 2; ++mm) {
       const int m = 2 * wave + mm;
@@ -331,19 +330,54 @@ __global__ __launch_bounds__(256, 3) void fwd_prep_kernel(
         f32x4 acc = zero4();
 #pragma unroll
         for (int kb = 0; kb < 2; ++kb) acc = mfma(ak[kb], ld8(Ts + (16 * n + r) * LDT + 32 * kb + 8 * q4), acc);
-        // row t = 16 n + r (rows past the chunk fall outside w_rs)
-        __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, to4<E>(-acc)), w_rs,
-                                              r * rowe + perm32(16 * m + 4 * q4) * (int)sizeof(E), 16 * n * rowe, 0);
+        wo[mm][n] = to4<E>(-acc);
       }
     }
   }
-  __syncthreads();
+  // The outputs leave as whole rows through LDS (a store whose lanes are rows takes the
+  // vector memory unit 2.5 times as long; with V read by row pieces instead of column
+  // gathers: H = 16, 144 / 520 / 36 / 5 chunks 60.0 -> 51.5 / 198 -> 154 / 21.0 -> 19.1 /
+  // 13.2 -> 11.9 us, 4.1 and 4.9 TB/s on the two long ones): Kg^T from the solve's region, -W through the
+  // K rows' place, then U^T through the solve's region.
+  __syncthreads();  // the KgT tile is complete, every read of beta gam K is done
   {
     E* kgt = KgT + cb * (D * CH);
+    X8 x[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int seg = 256 * i + tid;
-      st8(kgt + seg * 8, ld8(kgs + (seg ^ (((seg >> 4) & 3) + 4 * ((seg >> 3) & 1))) * 8));
+      x[i] = ld8(kgs + (seg ^ (((seg >> 4) & 3) + 4 * ((seg >> 3) & 1))) * 8);
+    }
+#pragma unroll
+    for (int mm = 0; mm < 2; ++mm)  // row t = 16 n + r, columns k = 16 (2 wave + mm) + 4 q4 .. in perm32 order
+#pragma unroll
+      for (int n = 0; n < 4; ++n)
+        *reinterpret_cast<X4*>(Ks + (16 * n + r) * LDK + perm32(16 * (2 * wave + mm) + 4 * q4)) = wo[mm][n];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) st8(kgt + (256 * i + tid) * 8, x[i]);
+  }
+  lds_barrier();  // every read of the KgT tile is done, -W is complete
+  {
+    const __amdgpu_buffer_rsrc_t w_rs = buf_rsrc(W + ((size_t)ci.start * H + h) * D, rows_bytes);
+    X8 x[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) x[j] = ld8(Ks + t_r * LDK + 32 * j + 8 * p_r);
+#pragma unroll
+    for (int nn = 0; nn < 2; ++nn)  // U^T row v = 16 (2 wave + nn) + r, t = 16 tt + 4 q4 ..
+#pragma unroll
+      for (int tt = 0; tt < 4; ++tt)
+        *reinterpret_cast<X4*>(kgs + (16 * (2 * wave + nn) + r) * CH + 8 * ((2 * tt + (q4 >> 1)) ^ (r & 7)) + 4 * (q4 & 1)) =
+            uo[nn][tt];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) buf_st16(w_rs, t_r * rowe + 64 * j + 16 * p_r, x[j]);  // rows past the chunk fall outside w_rs
+  }
+  lds_barrier();
+  {
+    E* ut = UT + cb * (D * CH);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int seg = 256 * i + tid;  // row v = seg / 8, 16-byte column seg % 8
+      st8(ut + seg * 8, ld8(kgs + (seg ^ ((seg >> 3) & 7)) * 8));
     }
   }
   if (SCALED && blockIdx.x == 0 && blockIdx.y == 0 && tid == 0) vscale[0] = vs;
