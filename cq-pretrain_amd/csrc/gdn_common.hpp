@@ -252,6 +252,15 @@ template <class T>  // bf16 or f16
 __device__ __forceinline__ typename Vec<T>::x8 row_piece(const T* M, size_t ld, int row, int c0) {
   return ld8(M + row * ld + c0 + 8 * (threadIdx.x & 3));
 }
+// The same for an operand that runs along M's rows: x is 16 rows read by row_piece (32
+// columns), and lane (q4, r) gets row r, columns 8 q4 .. 8 q4 + 7 (what ld8 from lane r on
+// row r reads at a third of the rate), through 1 KB of LDS of the wave's own.
+template <class T>
+__device__ __forceinline__ typename Vec<T>::x8 operand_from_rows(T* own, typename Vec<T>::x8 x) {
+  const int lane = threadIdx.x & 63, r = lane & 15, q4 = lane >> 4;
+  st8(own + (lane >> 2) * 32 + 8 * ((lane & 3) ^ ((lane >> 3) & 3)), x);
+  return ld8(own + r * 32 + 8 * (q4 ^ ((r >> 1) & 3)));
+}
 template <class T>
 __device__ __forceinline__ void columns_from_rows(T* own, typename Vec<T>::x8 x0, typename Vec<T>::x8 x1,
                                                   typename Vec<T>::x8 (&y)[2]) {

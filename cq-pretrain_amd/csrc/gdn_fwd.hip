@@ -595,7 +595,11 @@ __global__ __launch_bounds__(SCAN_THREADS, 2) void fwd_scan_kernel(
 }
 
 // ---------------------------------------------------------------------------
-// fwd_out: O^T (v rows, t columns) per chunk and head.
+// fwd_out: O^T (v rows, t columns) per chunk and head.  h^T and v_new^T come in by row
+// pieces (operand_from_rows) and O leaves as whole rows: H = 16, 144 / 520 / 36 / 5 chunks
+// 46.6 -> 43.6 / 152.7 -> 146.8 / 16.5 -> 15.9 / 7.9 -> 7.2 us against fragments read and
+// O stored with lanes on 16 different rows.  Bound by HBM on the long ones: 222 MB at 5.1
+// TB/s (a large copy reaches 5.2).
 // ---------------------------------------------------------------------------
 template <class I, class E>  // I: element type of q, k and o; E: operand type (as fwd_prep)
 __global__ __launch_bounds__(256) void fwd_out_kernel(
@@ -620,15 +624,16 @@ __global__ __launch_bounds__(256) void fwd_out_kernel(
 
   const E* ht = hT + cb * (D * D);
   const E* vt = vnT + cb * (D * CH);
-  // requested with the inputs: rows v = 16 (2 wave + mm) + r of v_new^T (t block
+  // requested with the inputs, by quads: rows v = 16 (2 wave + mm) .. of v_new^T (t block
   // kb) and of h^T (k block kb)
   X8 av[2][2], ah[2][4];
 #pragma unroll
   for (int mm = 0; mm < 2; ++mm) {
+    const int v = 16 * (2 * wave + mm) + (lane >> 2);
 #pragma unroll
-    for (int kb = 0; kb < 2; ++kb) av[mm][kb] = ld8(vt + (16 * (2 * wave + mm) + r) * CH + 32 * kb + 8 * q4);
+    for (int kb = 0; kb < 2; ++kb) av[mm][kb] = row_piece(vt, CH, v, 32 * kb);
 #pragma unroll
-    for (int kb = 0; kb < 4; ++kb) ah[mm][kb] = ld8(ht + (16 * (2 * wave + mm) + r) * D + 32 * kb + 8 * q4);
+    for (int kb = 0; kb < 4; ++kb) ah[mm][kb] = row_piece(ht, D, v, 32 * kb);
   }
   {
     const int t = tid >> 2, p = tid & 3;
@@ -650,6 +655,14 @@ __global__ __launch_bounds__(256) void fwd_out_kernel(
       st8(Qs + t * LDK + col, keep_if(in, scaled8<E>(xq[j], rqt)));
       st8(Ks + t * LDK + col, keep_if(in, scaled8<E>(xk[j], rkt)));
     }
+  }
+  // to the operands' layout through the place of P
+#pragma unroll
+  for (int mm = 0; mm < 2; ++mm) {
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb) av[mm][kb] = operand_from_rows(Ps + 1024 * wave + 512 * (kb & 1), av[mm][kb]);
+#pragma unroll
+    for (int kb = 0; kb < 4; ++kb) ah[mm][kb] = operand_from_rows(Ps + 1024 * wave + 512 * (kb & 1), ah[mm][kb]);
   }
   __syncthreads();
 
@@ -709,14 +722,19 @@ __global__ __launch_bounds__(256) void fwd_out_kernel(
     }
   }
   const float osc = vscale ? scale / *vscale : scale;  // undo the power-of-two scale of V
+  // O leaves as whole rows, through the Q rows' place
+  static_assert(sizeof(I) == sizeof(E), "O rows fit the Q rows");
+  I* Os = reinterpret_cast<I*>(Qs);
+  lds_barrier();
 #pragma unroll
-  for (int n = 0; n < 4; ++n) {
-    const int t = 16 * n + r;
-    if (t >= ci.len) continue;
-    I* orow = o + ((size_t)(ci.start + t) * H + h) * D;
+  for (int n = 0; n < 4; ++n)
 #pragma unroll
-    for (int mm = 0; mm < 2; ++mm) st4(orow + 16 * (2 * wave + mm) + 4 * q4, acc[mm][n] * osc);
-  }
+    for (int mm = 0; mm < 2; ++mm) st4(Os + (16 * n + r) * LDK + 16 * (2 * wave + mm) + 4 * q4, acc[mm][n] * osc);
+  lds_barrier();
+  const __amdgpu_buffer_rsrc_t o_rs = chunk_rows_rsrc(o, ci.start, ci.len, H, h);
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+    buf_st16(o_rs, (tid >> 2) * H * D * 2 + 64 * j + 16 * (tid & 3), ld8(Os + (tid >> 2) * LDK + 32 * j + 8 * (tid & 3)));
 }
 
 // ---------------------------------------------------------------------------
