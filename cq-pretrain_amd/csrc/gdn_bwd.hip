@@ -271,10 +271,8 @@ __global__ __launch_bounds__(256, 3) void bwd_local_kernel(
 // so a lane's eight values of dS are consecutive in k: one 16-byte LDS write, and one
 // 16-byte piece of X^T.
 //
-// Measured (H = 16, one document of 144 chunks / 15 documents, 520 chunks): 116.6 -> 104.4
-// us, 331 -> 299 us; 36 chunks 32.4 -> 25.3; four heads, 144 chunks 113.6 -> 83.4; beside
-// bwd_dkw a step of 144 chunks went from 477 to 448 us, the scan (7 KB of LDS instead of
-// 152) now sharing its CUs with bwd_dkw workgroups.
+// Measured (H = 16, one document of 144 chunks / 15 documents, 520 chunks): 116.6 -> 92
+// us, 331 -> 290 us; 36 chunks 32.4 -> 24.2; four heads, 144 chunks 113.6 -> 77.9.
 //
 // The outputs are stored with the non-temporal hint: the scan still has the earlier chunks'
 // operands to read (bwd_local wrote them first to last, so they are the oldest in the
@@ -322,7 +320,8 @@ __global__ __launch_bounds__(SCAN_THREADS, 2) void bwd_scan_kernel(
   ScanTable tab(chunks, gc, nullptr, c_last, -1, n, H, h, lane);
   const size_t cb = (size_t)c_last * H + h;
   const int64_t tile = (int64_t)H * D * CH * 2;  // bytes from one chunk's [D][64] tile to the next chunk's
-  ScanBlocks<true> kb(knP + cb * (D * CH), tile, n), wb(WT + cb * (D * CH), tile, n);
+  ScanBlocks<true> kb(knP + cb * (D * CH), tile, n);
+  ScanBlocks<true> wb(WT + (cb + H) * (D * CH), tile, n + 1);  // one step behind: its first block is step -1's
   ScanBlocks<true> lb(dvlT + cb * (D * CH) + v0 * CH, tile, n), xb(XT + cb * (D * D) + v0 * D, 2 * tile, n);
   ScanBlocks<true> sb(dhS + cb * (D * D) + slice * (D * 16), 2 * tile, n);
   ScanBlocks<true> nb(dVnS + cb * (CH * D) + slice * (CH * 16), tile, n);
@@ -363,7 +362,7 @@ __global__ __launch_bounds__(SCAN_THREADS, 2) void bwd_scan_kernel(
 #pragma unroll
   for (int i = 0; i < SCAN_DEPTH; ++i) {
     issue_n(i, i);
-    issue_w(i, i);
+    if (i > 0) issue_w(i - 1, i);
   }
   kb.advance();
   wb.advance();
@@ -380,6 +379,7 @@ __global__ __launch_bounds__(SCAN_THREADS, 2) void bwd_scan_kernel(
 #pragma unroll
     for (int j = 1; j < 4; ++j) sx[j - 1] = ld8(Sx + r * SCAN_SROW + 32 * ((wave + j) & 3) + 8 * q4);
     const X8 ds_out = ld8_tr16(Sx, SCAN_SROW, 32 * wave);
+    if constexpr (decltype(more)::value) issue_w((s + SCAN_DEPTH - 1) % SCAN_DEPTH, s);
 #pragma unroll
     for (int j = 1; j < 4; ++j) acc = mfma(fn[s][j], sx[j - 1], acc);
     buf_st16<OUT>(sb.buffer(), s_out + sb.offset(s), ds_out);
@@ -402,7 +402,6 @@ __global__ __launch_bounds__(SCAN_THREADS, 2) void bwd_scan_kernel(
     for (int m = 0; m < 2; ++m) dS[m] = mfma(fw[s][m][0], b0, dS[m]);
 #pragma unroll
     for (int m = 0; m < 2; ++m) dS[m] = mfma(fw[s][m][1], b1, dS[m]);
-    if constexpr (decltype(more)::value) issue_w(s, s);
     buf_st8<OUT>(nb.buffer(), v_out, nb.offset(s), dv_out);
     own = to8<E>(f32x8{dS[0][0], dS[0][1], dS[0][2], dS[0][3], dS[1][0], dS[1][1], dS[1][2], dS[1][3]});
     st8(Sx + s_own, own);

@@ -411,20 +411,23 @@ __global__ __launch_bounds__(256, 3) void fwd_prep_kernel(
 //   slowed fwd_out by 3 us and gained nothing more on a step).
 // With fragments read straight from the row-major matrices the same kernel took 173 us.
 // Operands are requested SCAN_DEPTH steps ahead into registers (and four LDS rings);
-// 3, 5 or 6 steps measured the same.  No step computes an address (ScanBlocks, ScanTable)
+// 3, 5 or 6 steps measured the same.  Half of a step's requests go out in each of its
+// two waits (Kg^T a step later than -W): all at once they filled the memory unit's queue
+// and held up the wave's MFMAs (H = 16 / 4, 144 chunks: 84.5 -> 80.7 / 74.6 -> 72.8 us,
+// the reverse scan 93.4 -> 92 / 83.5 -> 77.9; 36 chunks 23.1 -> 22.0, 25.3 -> 24.2).  No step computes an address (ScanBlocks, ScanTable)
 // and nothing in a round is conditional, so the compiler's own waits leave every later
 // request in flight; the first round is peeled because a loop entered with fewer
 // operations in flight than it runs with waits as strictly as its entry.
 //
-// Measured (H = 16, one document of 144 chunks / 15 documents, 520 chunks): 102.6 -> 86.0
-// us, 294 -> 247 us; 36 chunks 29.1 -> 23.7; four heads, 144 chunks 97.9 -> 75.3.  LDS
+// Measured (H = 16, one document of 144 chunks / 15 documents, 520 chunks): 102.6 -> 80.7
+// us, 294 -> 240 us; 36 chunks 29.1 -> 22.0; four heads, 144 chunks 97.9 -> 72.8.  LDS
 // went from 136 KB to 72 KB a workgroup, so two share a CU.
 //
 // The waits for -W: loads, copies and stores of a wave retire in issue order, so a copy
 // has landed once at most as many operations are in flight as were surely issued after
 // it.  Counted are the operations of whole windows between barriers (the compiler may
-// reorder a window's own): a full step issues 11 (9 loads, 2 stores), and the store of
-// h^T precedes the wait.
+// reorder a window's own): a full step issues 11 (9 loads, 2 stores), and the Kg^T loads
+// and the store of h^T of its own step precede the wait.
 constexpr int FWD_STEP_OPS = 11, FWD_LOAD_OPS = 9;
 template <class E>
 __global__ __launch_bounds__(SCAN_THREADS, 2) void fwd_scan_kernel(
@@ -463,7 +466,8 @@ __global__ __launch_bounds__(SCAN_THREADS, 2) void fwd_scan_kernel(
     ScanTable tab(chunks, gc, W, c_begin, 1, n, H, h, lane);
     const size_t cb = (size_t)c_begin * H + h;
     const int64_t tile = (int64_t)H * D * CH * 2;  // bytes from one chunk's [D][64] tile to the next chunk's
-    ScanBlocks<false> kb(KgT + cb * (D * CH), tile, n), ub(UT + cb * (D * CH) + v0 * CH, tile, n);
+    ScanBlocks<false> ub(UT + cb * (D * CH) + v0 * CH, tile, n);
+    ScanBlocks<false> kb(KgT + (cb - H) * (D * CH), tile, n + 1);  // one step behind: its first block is step -1's
     ScanBlocks<false> vb(vnT + cb * (D * CH) + v0 * CH, tile, n), hb(hT + cb * (D * D) + v0 * D, 2 * tile, n);
     // per-lane parts of the addresses, the same for every chunk (bytes of global
     // memory; elements of LDS)
@@ -508,7 +512,7 @@ __global__ __launch_bounds__(SCAN_THREADS, 2) void fwd_scan_kernel(
 #pragma unroll
     for (int x = 0; x < SCAN_DEPTH; ++x) {
       issue_w(x, x);
-      issue_k(x, x);
+      if (x > 0) issue_k(x - 1, x);
       __builtin_amdgcn_sched_barrier(0);  // in this order: the waits count on it
     }
     // -W of the next step, once at most `flight` operations are in flight
@@ -534,6 +538,7 @@ __global__ __launch_bounds__(SCAN_THREADS, 2) void fwd_scan_kernel(
 #pragma unroll
       for (int j = 0; j < 4; ++j) sx[j] = ld8(Sx + s_in + 8 * j);
       const X8 h_out = cat(ld4(Sx + s_lo), ld4(Sx + s_hi));
+      if constexpr (decltype(more)::value) issue_k((s + SCAN_DEPTH - 1) % SCAN_DEPTH, s);
       f32x4 acc = cvtf4(u);
 #pragma unroll
       for (int j = 0; j < 4; ++j) acc = mfma(w[j], sx[j], acc);
@@ -553,10 +558,7 @@ __global__ __launch_bounds__(SCAN_THREADS, 2) void fwd_scan_kernel(
       for (int m = 0; m < 2; ++m) S[m] = mfma(fk[s][m][0], b0, S[m]);
 #pragma unroll
       for (int m = 0; m < 2; ++m) S[m] = mfma(fk[s][m][1], b1, S[m]);
-      if constexpr (decltype(more)::value) {
-        issue_w(s, s);
-        issue_k(s, s);
-      }
+      if constexpr (decltype(more)::value) issue_w(s, s);
       buf_st8(vb.buffer(), vn_off, vb.offset(s), v_out);
       st8(Sx + s_own, pack_permv<E>(S[0], S[1]));
       lds_barrier();
@@ -577,7 +579,7 @@ __global__ __launch_bounds__(SCAN_THREADS, 2) void fwd_scan_kernel(
     if (n >= SCAN_DEPTH) {
       // its first step's next -W has two more slots' loads after it and this step's store
       round(0, Int<2 * FWD_LOAD_OPS + 1>());
-      for (tau = SCAN_DEPTH; tau + SCAN_DEPTH <= n; tau += SCAN_DEPTH) round(tau, Int<2 * FWD_STEP_OPS + 1>());
+      for (tau = SCAN_DEPTH; tau + SCAN_DEPTH <= n; tau += SCAN_DEPTH) round(tau, Int<2 * FWD_STEP_OPS + 5>());
     }
     // the last steps issue their two stores only (and n < SCAN_DEPTH never issued more than the first loads)
     if (tau < n) step(Int<0>(), Int<0>(), Int<2 * FWD_LOAD_OPS + 1>());
