@@ -110,21 +110,24 @@ int scan_side(ScanSide** out) {
   return CQGDN_OK;
 }
 
-constexpr int kBesideMinChunks = 64;
+constexpr int kBesideMinChunks = 64, kBesideMinChunkHeads = 1280;
 
-// The side stream for a kernel beside a state scan, or null (*out) when that kernel
-// runs after the scan: each scan workgroup (one per head, 16-wide value slice and
-// document) holds a whole CU, and the kernel beside waits for the scan's chunks,
-// so every scan workgroup must be resident at once, leaving at least half of the
-// CUs to the kernel beside; `env` = "0" in the environment keeps the kernel after
-// the scan.
-int side_beside_scan(const char* env, int64_t T, int H, int64_t n_chunks, int n_docs, ScanSide** out) {
+// The side stream for bwd_dkw beside the reverse scan, or null (*out) when bwd_dkw runs
+// after it.  Each scan workgroup (one per head, 16-wide value slice and document) then has
+// a CU to itself, and bwd_dkw waits for the scan's chunks, so every scan workgroup must be
+// resident at once, leaving at least half of the CUs to bwd_dkw, and the documents must
+// average kBesideMinChunks chunks (below, the side stream's launches and events cost more
+// than the scan takes).  Of those calls it pays where bwd_dkw is long enough: beside / after
+// the scan, us a step: 576 chunk-heads (4 heads x 144) 257 / 248, 1152 (8 x 144) 316 / 315
+// and (8 x 2 x 72) 247 / 244, 1088 (16 x 68) 233 / 236, 2304 (16 x 144) 426 / 452, 4096
+// (8 x 512) 1028 / 1100.  CQGDN_DKW_BESIDE_SCAN in the environment: "0" keeps bwd_dkw after
+// the scan, "1" runs it beside wherever it fits.
+int side_beside_scan(int64_t T, int H, int64_t n_chunks, int n_docs, ScanSide** out) {
   *out = nullptr;
-  const char* e = getenv(env);
+  const char* e = getenv("CQGDN_DKW_BESIDE_SCAN");
   if ((e && e[0] == '0') || T <= 0 || H <= 0 || n_docs <= 0) return CQGDN_OK;
-  // documents of fewer chunks than this on average: the scan is too short for
-  // the side stream's extra launches and events to pay
   if (n_chunks < (int64_t)kBesideMinChunks * n_docs) return CQGDN_OK;
+  if (!(e && e[0] == '1') && n_chunks * H < kBesideMinChunkHeads) return CQGDN_OK;
   ScanSide* side = nullptr;
   if (const int err = scan_side(&side)) return err;
   if ((int64_t)H * 8 * n_docs * 2 <= side->cus) *out = side;
@@ -379,15 +382,13 @@ int cqgdn_bwd(const void* q, const void* k, const void* v, const float* g, const
               float scale, unsigned flags, const void* fwd_workspace, size_t fwd_workspace_bytes,
               void* bwd_workspace, size_t bwd_workspace_bytes, void* dq, void* dk, void* dv, float* dg, float* dbeta,
               void* stream) {
-  // bwd_dkw beside the reverse scan when every scan workgroup is resident at once
-  // (CQGDN_DKW_BESIDE_SCAN=0 keeps it after the scan); every argument is checked
-  // before the side stream is looked up
+  // every argument is checked before the side stream is looked up
   if (const int e = bwd_impl(q, k, v, g, beta, dout, T, H, chunk_table, n_chunks, doc_chunk, n_docs, scale, flags,
                              fwd_workspace, fwd_workspace_bytes, bwd_workspace, bwd_workspace_bytes, dq, dk, dv, dg,
                              dbeta, stream, false, nullptr))
     return e;
   ScanSide* side = nullptr;
-  if (const int e = side_beside_scan("CQGDN_DKW_BESIDE_SCAN", T, H, n_chunks, n_docs, &side)) return e;
+  if (const int e = side_beside_scan(T, H, n_chunks, n_docs, &side)) return e;
   return bwd_impl(q, k, v, g, beta, dout, T, H, chunk_table, n_chunks, doc_chunk, n_docs, scale, flags, fwd_workspace,
                   fwd_workspace_bytes, bwd_workspace, bwd_workspace_bytes, dq, dk, dv, dg, dbeta, stream, true,
                   nullptr, side ? side->stream : nullptr, side ? side->fork : nullptr, side ? side->join : nullptr);

@@ -286,6 +286,12 @@ __device__ __forceinline__ void bwd_publish(int* __restrict__ ready, int c, int 
   asm volatile("" ::: "memory");
 }
 
+// LDS that a scan workgroup with a bwd_dkw beside it takes in addition, unused: with it no
+// bwd_dkw workgroup (81 KB) shares its CU.  On a shared CU the two halve each other (H = 16,
+// 144 chunks: scan 180 us, step 432; alone on its CU 137 and 426; 512 chunks of 8 heads:
+// step 1064 and 1028).
+constexpr int BESIDE_LDS = 88 * 1024;
+
 // Vector memory operations of one full step of one wave: 8 operand fragments, X, dv_local,
 // two stores.  A step's chunk is announced BWD_ANNOUNCE steps later.
 constexpr int BWD_STEP_OPS = 12, BWD_ANNOUNCE = 3;
@@ -1228,7 +1234,8 @@ static hipError_t launch_bwd_t(const BwdArgs& a, hipStream_t stream) {
   {
     TimedLaunch tl(K_BWD_SCAN, stream);
     const auto kernel = beside ? bwd_scan_kernel<E, true> : bwd_scan_kernel<E, false>;
-    hipLaunchKernelGGL(kernel, dim3(a.H * (D / 16), a.n_docs), dim3(SCAN_THREADS), 0, stream, B(B_KNP), Ff(F_GC),
+    hipLaunchKernelGGL(kernel, dim3(a.H * (D / 16), a.n_docs), dim3(SCAN_THREADS), beside ? BESIDE_LDS : 0, stream,
+                       B(B_KNP), Ff(F_GC),
                        B(B_DVLT), B(B_XT), B(B_WT), a.chunks, a.doc_chunk, a.H, B(B_DH), B(B_DVN), ready, resident);
   }
   if (beside) {
