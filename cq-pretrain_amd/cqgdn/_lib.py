@@ -51,6 +51,7 @@ SIGNATURES = {
     "cqgdn_conv1d_fwd": (_I, [_P, _P, _P, _I, _I64, _I, _I, _I, _P, _P]),
     "cqgdn_conv1d_bwd_workspace_size": (_SZ, [_I64, _I, _I]),
     "cqgdn_conv1d_bwd": (_I, [_P, _P, _P, _P, _I, _I64, _I, _I, _I, _P, _P, _P, _SZ, _P]),
+    "cqgdn_prefill_cache": (_I, [_P, _I, _I, _I, _P, _I64, _P, _I, _I, _P, _P, _P]),
     "cqgdn_gated_norm_fwd": (_I, [_P, _P, _I64, _I, _P, _I64, _P, _F, _P, _P, _P]),
     "cqgdn_gated_norm_bwd_workspace_size": (_SZ, [_I64, _I]),
     "cqgdn_gated_norm_bwd": (_I, [_P, _P, _P, _I64, _I64, _I, _P, _I64, _P, _P, _P, _P, _P, _I64, _P, _P, _SZ, _P]),

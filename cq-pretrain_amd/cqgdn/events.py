@@ -283,13 +283,11 @@ def layer_prefill(proj, conv_weight, A_log, dt_bias, norm_weight, plan, *, heads
     rstd = torch.empty(n_h, heads, dtype=torch.float32, device=dev)
     gdn.call("cqgdn_gated_norm_fwd", gdn._ptr(y), gdn._ptr(ep.hidden_index), n_h, heads, proj[:, zc:].data_ptr(),
              P, gdn._ptr(nw), float(eps), gdn._ptr(out), gdn._ptr(rstd), st)
-    count = K - 1
-    history = proj.new_zeros(1, count, C)
-    order = ep.tensors["content_order"]
-    tail = order[max(0, ep.n_content - 1 - count):max(ep.n_content - 1, 0)].long()
-    if tail.numel():
-        history[0, count - tail.numel():] = proj.index_select(0, tail)[:, :C]
-    return out.reshape(n_h, S), {"state": state.transpose(-1, -2).contiguous(), "conv": history}
+    cache = {"state": torch.empty_like(state), "conv": torch.empty(1, K - 1, C, dtype=proj.dtype, device=dev)}
+    gdn.call("cqgdn_prefill_cache", gdn._ptr(state), state.shape[0], heads, HK, gdn._ptr(proj), P,
+             gdn._ptr(ep.tensors["content_order"]), ep.n_content, K, gdn._ptr(cache["state"]), gdn._ptr(cache["conv"]),
+             st)
+    return out.reshape(n_h, S), cache
 
 
 @torch.no_grad()

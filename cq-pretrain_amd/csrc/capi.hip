@@ -697,6 +697,29 @@ size_t cqgdn_layer_decode_workspace_size(int N, int H) {
   return 0;  // the step needs no workspace
 }
 
+int cqgdn_prefill_cache(const float* state, int n_docs, int H, int key_heads, const void* proj, int64_t proj_stride,
+                        const int32_t* content_order, int n_content, int conv_kernel, float* state_vk,
+                        void* history, void* stream) {
+  if (n_docs < 0 || n_content < 0) return fail(CQGDN_EINVAL, "n_docs and n_content must be >= 0");
+  if (head_group_shift(H, key_heads) < 0)
+    return fail(CQGDN_EINVAL, "H=%d key_heads=%d: supported local heads are 4, 8, 16, 32, key heads dividing H", H,
+                key_heads);
+  if (conv_kernel < 2 || conv_kernel > 4) return fail(CQGDN_EINVAL, "conv_kernel=%d not in 2..4", conv_kernel);
+  const int C = (2 * key_heads + H) * CQGDN_HEAD_DIM;
+  const int64_t states = (int64_t)n_docs * H;
+  if (states > (1 << 26)) return fail(CQGDN_EINVAL, "n_docs*H=%lld is too large", (long long)states);
+  if (states > 0 && (!state || !state_vk || !aligned(state, 16) || !aligned(state_vk, 16)))
+    return fail(CQGDN_EINVAL, "state and state_vk must be non-null and 16-byte aligned");
+  if (!history || !aligned(history, 16))
+    return fail(CQGDN_EINVAL, "history must be non-null and 16-byte aligned");
+  if (n_content > 1 && (!proj || !aligned(proj, 16) || !content_order || proj_stride < C || proj_stride % 8))
+    return fail(CQGDN_EINVAL, "proj (16-byte aligned, rows >= %d and a multiple of 8 elements apart) and content_order "
+                "must be non-null", C);
+  launch_prefill_cache(state, states, static_cast<const bf16*>(proj), proj_stride, C, content_order, n_content,
+                       conv_kernel - 1, state_vk, static_cast<bf16*>(history), (hipStream_t)stream);
+  return check_launch("cqgdn_prefill_cache");
+}
+
 int cqgdn_layer_decode_step(int N, int H, int key_heads, int conv_kernel, const void* proj, int64_t proj_stride,
                             void* conv_history, const void* conv_weight, const float* A_log, const float* dt_bias,
                             const float* norm_weight, float eps, float scale, float* state, void* out, void* workspace,

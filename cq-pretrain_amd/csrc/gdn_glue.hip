@@ -618,6 +618,44 @@ int gnorm_bwd_blocks(int64_t rows, int H) {
   return (int)(blocks < 1024 ? blocks : 1024);
 }
 
+// The decoder's cache after a prefill, in one launch (include/cqgdn.h).  Blocks [0, 16*states):
+// one 32x32 tile of a state each, read and written as whole 128-byte row pieces and turned in
+// LDS (rows of 33 floats: the column reads hit 32 banks).  The last `count` blocks: one history
+// row each.  Bound by its launch: one document of 16 heads is 1 MB each way.  torch's transpose,
+// row lookup, zero fill and two copies took 25 us in five launches there (137 us for the whole call); this takes 4.3 (120).
+__global__ __launch_bounds__(256) void prefill_cache_kernel(const float* __restrict__ state, int64_t tiles,
+                                                           const bf16* __restrict__ proj, int64_t proj_stride, int C,
+                                                           const int32_t* __restrict__ order, int n_content, int count,
+                                                           float* __restrict__ state_vk, bf16* __restrict__ history) {
+  const int64_t tile = blockIdx.x;
+  if (tile >= tiles) {
+    const int j = (int)(tile - tiles), pos = n_content - 1 - count + j;
+    const bf16* src = pos >= 0 ? proj + (int64_t)order[pos] * proj_stride : nullptr;
+    for (int c = 8 * threadIdx.x; c < C; c += 8 * 256)
+      *reinterpret_cast<bf16x8*>(history + (int64_t)j * C + c) =
+          src ? *reinterpret_cast<const bf16x8*>(src + c) : bf16x8{};
+    return;
+  }
+  __shared__ float turn[32][33];
+  const int64_t base = (tile / 16) * 128 * 128;
+  const int k0 = (int)(tile % 16) / 4 * 32, v0 = (int)(tile % 4) * 32, r = threadIdx.x / 8, c = threadIdx.x % 8 * 4;
+  const f32x4 x = *reinterpret_cast<const f32x4*>(state + base + (k0 + r) * 128 + v0 + c);
+#pragma unroll
+  for (int e = 0; e < 4; ++e) turn[r][c + e] = x[e];
+  __syncthreads();
+  f32x4 y;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) y[e] = turn[c + e][r];
+  *reinterpret_cast<f32x4*>(state_vk + base + (v0 + r) * 128 + k0 + c) = y;
+}
+
+void launch_prefill_cache(const float* state, int64_t states, const bf16* proj, int64_t proj_stride, int C,
+                          const int32_t* order, int n_content, int count, float* state_vk, bf16* history,
+                          hipStream_t stream) {
+  hipLaunchKernelGGL(prefill_cache_kernel, dim3((unsigned)(16 * states + count)), dim3(256), 0, stream, state,
+                     16 * states, proj, proj_stride, C, order, n_content, count, state_vk, history);
+}
+
 void launch_gnorm_fwd(const bf16* y, const int32_t* index, int64_t rows, int H, const bf16* z, int64_t z_stride,
                       const float* w, float eps, bf16* out, float* rstd, hipStream_t stream) {
   const int64_t items = rows * H;

@@ -165,6 +165,9 @@ void launch_decode_step(const DecArgs& a, float* state, const float* norm_w, flo
                         hipStream_t stream);
 // gated RMSNorm over D = 128 with an optional row gather (gdn_glue.hip)
 int gnorm_bwd_blocks(int64_t rows, int H);  // workgroups of the backward (dw partials per workgroup)
+void launch_prefill_cache(const float* state, int64_t states, const bf16* proj, int64_t proj_stride, int C,
+                          const int32_t* order, int n_content, int count, float* state_vk, bf16* history,
+                          hipStream_t stream);
 void launch_gnorm_fwd(const bf16* y, const int32_t* index, int64_t rows, int H, const bf16* z, int64_t z_stride,
                       const float* w, float eps, bf16* out, float* rstd, hipStream_t stream);
 void launch_gnorm_bwd(const bf16* y, const int32_t* index, const int32_t* zero_rows, int64_t n_zero, int64_t rows,

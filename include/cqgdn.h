@@ -224,6 +224,20 @@ int cqgdn_conv1d_bwd(const void* x, const void* weight, const void* dy, const in
                      void* stream);
 
 /*
+ * The cache a decoder continues from after a prefill (models/backbone_qwen35.py:163-211
+ * with ``cache``), in one launch.  state_vk fp32 [n_docs][H][128][128] receives each
+ * final state value-first (state_vk[i][h][v][k] = state[i][h][k][v]; the two must not
+ * overlap).  history bf16 [conv_kernel - 1][C], C = (2*key_heads + H)*128, receives the
+ * first C channels of the projection rows content_order[n_content - conv_kernel ..
+ * n_content - 2], zeros where the position is below 0.  proj: bf16 rows proj_stride
+ * elements apart (a multiple of 8, >= C); content_order: device int32 [n_content], each a
+ * row of proj, may be NULL if n_content < 2; conv_kernel: 2..4.
+ */
+int cqgdn_prefill_cache(const float* state, int n_docs, int H, int key_heads, const void* proj, int64_t proj_stride,
+                        const int32_t* content_order, int n_content, int conv_kernel, float* state_vk,
+                        void* history, void* stream);
+
+/*
  * Gated RMSNorm over D = 128 fused with the layer's output gather.  Replaces
  * gated_norm() (ops/gated_delta_net.py:67-74; CPU form GatedNorm.forward,
  * models/backbone_qwen35.py:107-114) applied to y.index_select(0, hidden_event)
