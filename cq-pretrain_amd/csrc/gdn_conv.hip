@@ -111,18 +111,22 @@ __global__ __launch_bounds__(CONV_THREADS) void conv_fwd_kernel(const bf16* __re
   }
 }
 
-// Backward: a one-wave workgroup streams a strip of rows [s, e) for
-// 64 * CONV_BWD_CH channels, walking u = s - (K-1) .. e + K - 2 in groups of K rows whose x and
-// dy rows are requested while the previous group computes.  Per row u:
+// Backward: a wave streams a strip of rows [s, e) for 64 * CONV_BWD_CH channels, walking u = s - (K-1) .. e + K - 2 in groups of K rows whose x and
+// dy rows are requested while the previous group computes (a gathered x row's index
+// one group before that).  Per row u:
 //   pre[u] from the last K x rows, dpre[u] = dy[u] * silu'(pre[u]),
 //   dw partials over u in [s, e),
 //   dx[t] = sum_j w[K-1-j] * dpre[t + j] over rows t + j of t's document.
 // The last K x rows (fp32) and dpre rows sit in rings indexed by the row's
 // place in its group, so the windows advance without register moves.  A strip
 // whose rows u0 .. uend-1 hold no document boundary (0 and T included) runs
-// without any per-row document test (DOCS = false).  Each strip writes its dw
-// partials [C][K]; colsum_kernel sums them.
+// without any per-row document test (DOCS = false).  A workgroup is four
+// neighbouring strips, whose rows overlap by K - 1 on each side: it sums their dw
+// partials in LDS, in strip order, and writes one [C][K] part; colsum_kernel sums
+// the parts.  Bound by the memory traffic: 8192 rows of 6144 channels take 65.7 us (58 at a large copy's rate),
+// 2048 rows 23.5; a one-wave workgroup and a part per strip took 69.7 and 25.5.
 constexpr int CONV_STRIPS = 128;  // row strips per 64 * CONV_BWD_CH channels
+constexpr int CONV_BWD_WAVES = 4; // strips per workgroup
 constexpr int CONV_BWD_CH = 4;    // channels per thread in the backward
 
 template <int CH> struct ConvVec;
@@ -140,12 +144,22 @@ __device__ __forceinline__ void conv_bwd_strip(const bf16* __restrict__ x, const
   typedef typename ConvVec<CH>::f fv;
   const int u0 = s - (K - 1), uend = e + K - 1;
   bv nx[K], nd[K];  // the next group's rows (clamped into [0, T); rows outside are never used)
+  int nr[K];        // the x rows of the group after it
+  auto place = [&](int u) { return min(max(u, 0), T - 1); };
+  auto index = [&](int ub) {
 #pragma unroll
-  for (int j = 0; j < K; ++j) {
-    const int u = min(max(u0 + j, 0), T - 1);
-    nx[j] = *reinterpret_cast<const bv*>(x + (rows ? (int64_t)rows[u] : (int64_t)u) * xstr + c);
-    nd[j] = *reinterpret_cast<const bv*>(dy + (int64_t)u * C + c);
-  }
+    for (int j = 0; j < K; ++j) nr[j] = rows ? rows[place(ub + j)] : place(ub + j);
+  };
+  auto request = [&](int ub) {
+#pragma unroll
+    for (int j = 0; j < K; ++j) {
+      nx[j] = *reinterpret_cast<const bv*>(x + (int64_t)nr[j] * xstr + c);
+      nd[j] = *reinterpret_cast<const bv*>(dy + (int64_t)place(ub + j) * C + c);
+    }
+    index(ub + K);
+  };
+  index(u0);
+  request(u0);
   // ring slot j holds the row at place j of the current group (rows before u0 are never read)
   fv xs[K], dp[K];
   int st[K];  // document start of each dpre ring row (-1: no row)
@@ -162,14 +176,7 @@ __device__ __forceinline__ void conv_bwd_strip(const bf16* __restrict__ x, const
       cx[j] = nx[j];
       cd[j] = nd[j];
     }
-    if (ub + K < uend) {
-#pragma unroll
-      for (int j = 0; j < K; ++j) {
-        const int u = min(max(ub + K + j, 0), T - 1);
-        nx[j] = *reinterpret_cast<const bv*>(x + (rows ? (int64_t)rows[u] : (int64_t)u) * xstr + c);
-        nd[j] = *reinterpret_cast<const bv*>(dy + (int64_t)u * C + c);
-      }
-    }
+    if (ub + K < uend) request(ub + K);
 #pragma unroll
     for (int j = 0; j < K; ++j) {
       const int u = ub + j;
@@ -219,35 +226,45 @@ __device__ __forceinline__ void conv_bwd_strip(const bf16* __restrict__ x, const
 }
 
 template <int K>
-__global__ __launch_bounds__(64) void conv_bwd_kernel(const bf16* __restrict__ x, const int32_t* __restrict__ xrows,
-                                                     int64_t xs, const bf16* __restrict__ w,
-                                                     const bf16* __restrict__ dy, const int32_t* __restrict__ bounds,
-                                                     int n_docs, int T, int C, int rows, int act,
-                                                     bf16* __restrict__ dx, const int32_t* __restrict__ dxrows,
-                                                     int64_t dxs, float* __restrict__ dw_part) {
+__global__ __launch_bounds__(64 * CONV_BWD_WAVES) void conv_bwd_kernel(
+    const bf16* __restrict__ x, const int32_t* __restrict__ xrows, int64_t xs, const bf16* __restrict__ w,
+    const bf16* __restrict__ dy, const int32_t* __restrict__ bounds, int n_docs, int T, int C, int rows, int act,
+    bf16* __restrict__ dx, const int32_t* __restrict__ dxrows, int64_t dxs, float* __restrict__ dw_part) {
   constexpr int CH = CONV_BWD_CH;
   typedef typename ConvVec<CH>::f fv;
-  const int c = (blockIdx.y * 64 + threadIdx.x) * CH;
-  if (c >= C) return;
-  const int s = blockIdx.x * rows, e = min(s + rows, T);
-  fv wk[K], dwa[K];
-  {
+  __shared__ fv red[CONV_BWD_WAVES - 1][K][64];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int c = (blockIdx.y * 64 + lane) * CH;
+  const int s = (blockIdx.x * CONV_BWD_WAVES + wave) * rows, e = min(s + rows, T);
+  fv dwa[K];
+#pragma unroll
+  for (int i = 0; i < K; ++i) dwa[i] = fv{};
+  if (c < C && s < T) {
+    fv wk[K];
     const bf16* wc = w + (size_t)c * K;
 #pragma unroll
     for (int ch = 0; ch < CH; ++ch)
 #pragma unroll
       for (int i = 0; i < K; ++i) wk[i][ch] = (float)wc[ch * K + i];
+    // a boundary b with u0 < b < uend separates two rows of the walk (b = 0 and b = T included)
+    const int u0 = s - (K - 1), uend = e + K - 1;
+    const int i = lower_bound(bounds, n_docs, u0 + 1);
+    const bool docs = __builtin_amdgcn_readfirstlane(i <= n_docs && bounds[i] < uend);
+    if (docs)
+      conv_bwd_strip<K, CH, true>(x, xrows, xs, wk, dy, bounds, n_docs, T, C, c, s, e, act, dx, dxrows, dxs, dwa);
+    else
+      conv_bwd_strip<K, CH, false>(x, xrows, xs, wk, dy, bounds, n_docs, T, C, c, s, e, act, dx, dxrows, dxs, dwa);
   }
+  if (wave > 0) {
 #pragma unroll
-  for (int i = 0; i < K; ++i) dwa[i] = fv{};
-  // a boundary b with u0 < b < uend separates two rows of the walk (b = 0 and b = T included)
-  const int u0 = s - (K - 1), uend = e + K - 1;
-  const int i = lower_bound(bounds, n_docs, u0 + 1);
-  const bool docs = __builtin_amdgcn_readfirstlane(i <= n_docs && bounds[i] < uend);
-  if (docs)
-    conv_bwd_strip<K, CH, true>(x, xrows, xs, wk, dy, bounds, n_docs, T, C, c, s, e, act, dx, dxrows, dxs, dwa);
-  else
-    conv_bwd_strip<K, CH, false>(x, xrows, xs, wk, dy, bounds, n_docs, T, C, c, s, e, act, dx, dxrows, dxs, dwa);
+    for (int i = 0; i < K; ++i) red[wave - 1][i][lane] = dwa[i];
+  }
+  __syncthreads();
+  if (wave > 0 || c >= C) return;
+#pragma unroll
+  for (int v = 0; v < CONV_BWD_WAVES - 1; ++v)
+#pragma unroll
+    for (int i = 0; i < K; ++i) dwa[i] += red[v][i][lane];
   float* part = dw_part + ((size_t)blockIdx.x * C + c) * K;
 #pragma unroll
   for (int ch = 0; ch < CH; ++ch)
@@ -290,8 +307,8 @@ __global__ __launch_bounds__(256) void colsum_kernel(const float* __restrict__ p
 
 int conv_strip_rows(int64_t T) { return (int)std::max<int64_t>(16, (T + CONV_STRIPS - 1) / CONV_STRIPS); }
 
-int conv_strips(int64_t T) {
-  const int64_t rows = conv_strip_rows(T);
+int conv_parts(int64_t T) {
+  const int64_t rows = (int64_t)conv_strip_rows(T) * CONV_BWD_WAVES;
   return (int)((T + rows - 1) / rows);
 }
 
@@ -308,14 +325,14 @@ void launch_conv_fwd(const bf16* x, const int32_t* xrows, int64_t xs, const bf16
 void launch_conv_bwd(const bf16* x, const int32_t* xrows, int64_t xs, const bf16* w, const bf16* dy,
                      const int32_t* bounds, int n_docs, int T, int C, int K, int act, bf16* dx, const int32_t* dxrows,
                      int64_t dxs, float* dw, float* part, hipStream_t stream) {
-  const int rows = conv_strip_rows(T), strips = conv_strips(T);
-  const dim3 grid(strips, (C / CONV_BWD_CH + 63) / 64);
+  const int rows = conv_strip_rows(T), parts = conv_parts(T);
+  const dim3 grid(parts, (C / CONV_BWD_CH + 63) / 64), block(64 * CONV_BWD_WAVES);
   switch (K) {
-    case 2: hipLaunchKernelGGL(conv_bwd_kernel<2>, grid, dim3(64), 0, stream, x, xrows, xs, w, dy, bounds, n_docs, T, C, rows, act, dx, dxrows, dxs, part); break;
-    case 3: hipLaunchKernelGGL(conv_bwd_kernel<3>, grid, dim3(64), 0, stream, x, xrows, xs, w, dy, bounds, n_docs, T, C, rows, act, dx, dxrows, dxs, part); break;
-    default: hipLaunchKernelGGL(conv_bwd_kernel<4>, grid, dim3(64), 0, stream, x, xrows, xs, w, dy, bounds, n_docs, T, C, rows, act, dx, dxrows, dxs, part); break;
+    case 2: hipLaunchKernelGGL(conv_bwd_kernel<2>, grid, block, 0, stream, x, xrows, xs, w, dy, bounds, n_docs, T, C, rows, act, dx, dxrows, dxs, part); break;
+    case 3: hipLaunchKernelGGL(conv_bwd_kernel<3>, grid, block, 0, stream, x, xrows, xs, w, dy, bounds, n_docs, T, C, rows, act, dx, dxrows, dxs, part); break;
+    default: hipLaunchKernelGGL(conv_bwd_kernel<4>, grid, block, 0, stream, x, xrows, xs, w, dy, bounds, n_docs, T, C, rows, act, dx, dxrows, dxs, part); break;
   }
-  launch_colsum(part, strips, C * K, dw, stream);
+  launch_colsum(part, parts, C * K, dw, stream);
 }
 
 // The same sums for few columns (n % 4 == 0) and many parts: a workgroup of 1024 threads

@@ -73,7 +73,7 @@ void launch_recurrent(const void* q, const void* k, const void* v, const float* 
                       bool beta_bf16, bool fp16, float* state, void* out, int N, int E, int H, float scale,
                       hipStream_t stream);
 // packed depthwise causal conv1d (gdn_conv.hip); bounds: int32 [n_docs + 1] on the device
-int conv_strips(int64_t T);  // row strips of the conv backward (dw partials per strip)
+int conv_parts(int64_t T);  // workgroups along the rows of the conv backward (a dw partial each)
 // x row u is x + (xrows ? xrows[u] : u) * xs; dx row t is dx + (dxrows ? dxrows[t] : t) * dxs; y and dy are [T][C]
 void launch_conv_fwd(const bf16* x, const int32_t* xrows, int64_t xs, const bf16* w, const int32_t* bounds,
                      int n_docs, int T, int C, int K, int act, bf16* y, hipStream_t stream);
