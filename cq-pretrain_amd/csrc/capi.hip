@@ -629,7 +629,7 @@ int cqgdn_event_inputs_fwd(const cqgdn_event_plan* plan, int H, int key_heads, c
 
 namespace {
 struct EvLayout {
-  size_t dconv, dpre, gpart, qpart, cpart, qsum, dcont, dcgate, total;
+  size_t dconv, dpre, gpart, qpart, cpart, dcont, dcgate, total;
 };
 EvLayout ev_layout(int n_content, int n_queries, int H, int HK, int K, bool fold) {
   const size_t SK = (size_t)HK * CQGDN_HEAD_DIM, C = 2 * SK + (size_t)H * CQGDN_HEAD_DIM;
@@ -642,7 +642,6 @@ EvLayout ev_layout(int n_content, int n_queries, int H, int HK, int K, bool fold
   l.gpart = o; o += align256((size_t)n_content * 2 * H * sizeof(float));
   l.qpart = o; o += align256((size_t)events_query_blocks(n_queries) * SK * K * sizeof(float));
   l.cpart = o; o += align256((size_t)(n_content > 0 ? conv_parts(n_content) : 0) * C * K * sizeof(float));
-  l.qsum = o; o += align256(SK * K * sizeof(float));
   l.total = o + 256;
   return l;
 }
@@ -686,7 +685,7 @@ int cqgdn_event_inputs_bwd(const cqgdn_event_plan* plan, int H, int key_heads, c
                   plan->fold_ptr, plan->fold_list};
   const EvWork w{reinterpret_cast<bf16*>(ws + l.dconv), reinterpret_cast<float*>(ws + l.dpre),
                  reinterpret_cast<float*>(ws + l.gpart), reinterpret_cast<float*>(ws + l.qpart),
-                 reinterpret_cast<float*>(ws + l.cpart), reinterpret_cast<float*>(ws + l.qsum)};
+                 reinterpret_cast<float*>(ws + l.cpart)};
   launch_events_bwd(ea, d, plan->content_bounds, plan->n_content_docs, w, (hipStream_t)stream);
   return check_launch("cqgdn_event_inputs_bwd");
 }

@@ -276,7 +276,9 @@ __global__ __launch_bounds__(64 * CONV_BWD_WAVES) void conv_bwd_kernel(
 // and the other per-workgroup parameter-gradient partials): a lane owns 4
 // consecutive j (16-byte loads), a workgroup 256 j; its 4 waves sum strips
 // b = wave, wave + 4, ... with 8 loads in flight, and the four sums are added
-// in wave order (fixed order: deterministic).
+// in wave order (fixed order: deterministic).  ADD: dw[j] += that sum (in place of a launch
+// of its own for the addition).
+template <bool ADD>
 __global__ __launch_bounds__(256) void colsum_kernel(const float* __restrict__ part, int strips, int n,
                                                     float* __restrict__ dw) {
   __shared__ f32x4 red[4][64];
@@ -301,7 +303,7 @@ __global__ __launch_bounds__(256) void colsum_kernel(const float* __restrict__ p
   if (wave == 0 && j < n) {
     const f32x4 r = ((red[0][lane] + red[1][lane]) + red[2][lane]) + red[3][lane];
 #pragma unroll
-    for (int q = 0; q < 4; ++q) dw[j + q] = r[q];
+    for (int q = 0; q < 4; ++q) dw[j + q] = ADD ? dw[j + q] + r[q] : r[q];
   }
 }
 
@@ -375,7 +377,12 @@ void launch_colsum(const float* part, int parts, int n, float* out, hipStream_t 
   if (n <= 256 && parts > 64)
     hipLaunchKernelGGL(colsum_narrow_kernel, dim3((n + 15) / 16), dim3(1024), 0, stream, part, parts, n, out);
   else
-    hipLaunchKernelGGL(colsum_kernel, dim3((n / 4 + 63) / 64), dim3(256), 0, stream, part, parts, n, out);
+    hipLaunchKernelGGL(colsum_kernel<false>, dim3((n / 4 + 63) / 64), dim3(256), 0, stream, part, parts, n, out);
+}
+
+void launch_colsum_add(const float* part, int parts, int n, float* out, hipStream_t stream) {
+  if (parts > 0)
+    hipLaunchKernelGGL(colsum_kernel<true>, dim3((n / 4 + 63) / 64), dim3(256), 0, stream, part, parts, n, out);
 }
 
 }  // namespace cqgdn

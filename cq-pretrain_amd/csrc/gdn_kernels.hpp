@@ -82,6 +82,7 @@ void launch_conv_bwd(const bf16* x, const int32_t* xrows, int64_t xs, const bf16
                      int64_t dxs, float* dw, float* part, hipStream_t stream);
 // out[j] = sum over p < parts of part[p][j], fixed order (gdn_conv.hip); n % 4 == 0, 16-byte aligned part
 void launch_colsum(const float* part, int parts, int n, float* out, hipStream_t stream);
+void launch_colsum_add(const float* part, int parts, int n, float* out, hipStream_t stream);  // out += the sums
 // Event inputs of one GatedDelta layer (gdn_glue.hip).  S = H * 128 channels per
 // q/k/v part; index arrays are device int32 (content rows are 0 .. n_c-1, n_c is
 // the zero row / "none").
@@ -142,7 +143,6 @@ struct EvWork {
   float* gpart;  // [n_c][2H]
   float* qpart;  // [events_query_blocks][SK][K]
   float* cpart;  // conv backward partials
-  float* qsum;   // [SK][K]
 };
 int events_query_blocks(int n_q);
 void launch_events_fwd(const EvArgs& a, const bf16* conv, bf16* q, bf16* k, bf16* v, float* g, float* beta,
