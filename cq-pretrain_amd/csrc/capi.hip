@@ -500,7 +500,8 @@ int cqgdn_conv1d_bwd(const void* x, const void* weight, const void* dy, const in
     return fail(CQGDN_EINVAL, "workspace must be 16-byte aligned and >= cqgdn_conv1d_bwd_workspace_size bytes");
   launch_conv_bwd(static_cast<const bf16*>(x), nullptr, C, static_cast<const bf16*>(weight),
                   static_cast<const bf16*>(dy), bounds, n_docs, (int)T, C, K, activation != 0, static_cast<bf16*>(dx),
-                  nullptr, C, dweight, static_cast<float*>(workspace), (hipStream_t)stream);
+                  nullptr, C, static_cast<float*>(workspace), (hipStream_t)stream);
+  launch_colsum(static_cast<const float*>(workspace), conv_parts(T), C * K, dweight, (hipStream_t)stream);
   return check_launch("cqgdn_conv1d_bwd");
 }
 

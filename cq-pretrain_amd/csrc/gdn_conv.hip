@@ -122,8 +122,8 @@ __global__ __launch_bounds__(CONV_THREADS) void conv_fwd_kernel(const bf16* __re
 // whose rows u0 .. uend-1 hold no document boundary (0 and T included) runs
 // without any per-row document test (DOCS = false).  A workgroup is four
 // neighbouring strips, whose rows overlap by K - 1 on each side: it sums their dw
-// partials in LDS, in strip order, and writes one [C][K] part; colsum_kernel sums
-// the parts.  Bound by the memory traffic: 8192 rows of 6144 channels take 65.7 us (58 at a large copy's rate),
+// partials in LDS, in strip order, and writes one [C][K] part; colsum_kernel (event_sums_kernel in a layer)
+// sums the parts.  Bound by the memory traffic: 8192 rows of 6144 channels take 65.7 us (58 at a large copy's rate),
 // 2048 rows 23.5; a one-wave workgroup and a part per strip took 69.7 and 25.5.
 constexpr int CONV_STRIPS = 128;  // row strips per 64 * CONV_BWD_CH channels
 constexpr int CONV_BWD_WAVES = 4; // strips per workgroup
@@ -276,9 +276,7 @@ __global__ __launch_bounds__(64 * CONV_BWD_WAVES) void conv_bwd_kernel(
 // and the other per-workgroup parameter-gradient partials): a lane owns 4
 // consecutive j (16-byte loads), a workgroup 256 j; its 4 waves sum strips
 // b = wave, wave + 4, ... with 8 loads in flight, and the four sums are added
-// in wave order (fixed order: deterministic).  ADD: dw[j] += that sum (in place of a launch
-// of its own for the addition).
-template <bool ADD>
+// in wave order (fixed order: deterministic).
 __global__ __launch_bounds__(256) void colsum_kernel(const float* __restrict__ part, int strips, int n,
                                                     float* __restrict__ dw) {
   __shared__ f32x4 red[4][64];
@@ -303,7 +301,7 @@ __global__ __launch_bounds__(256) void colsum_kernel(const float* __restrict__ p
   if (wave == 0 && j < n) {
     const f32x4 r = ((red[0][lane] + red[1][lane]) + red[2][lane]) + red[3][lane];
 #pragma unroll
-    for (int q = 0; q < 4; ++q) dw[j + q] = ADD ? dw[j + q] + r[q] : r[q];
+    for (int q = 0; q < 4; ++q) dw[j + q] = r[q];
   }
 }
 
@@ -326,7 +324,7 @@ void launch_conv_fwd(const bf16* x, const int32_t* xrows, int64_t xs, const bf16
 
 void launch_conv_bwd(const bf16* x, const int32_t* xrows, int64_t xs, const bf16* w, const bf16* dy,
                      const int32_t* bounds, int n_docs, int T, int C, int K, int act, bf16* dx, const int32_t* dxrows,
-                     int64_t dxs, float* dw, float* part, hipStream_t stream) {
+                     int64_t dxs, float* part, hipStream_t stream) {
   const int rows = conv_strip_rows(T), parts = conv_parts(T);
   const dim3 grid(parts, (C / CONV_BWD_CH + 63) / 64), block(64 * CONV_BWD_WAVES);
   switch (K) {
@@ -334,18 +332,17 @@ void launch_conv_bwd(const bf16* x, const int32_t* xrows, int64_t xs, const bf16
     case 3: hipLaunchKernelGGL(conv_bwd_kernel<3>, grid, block, 0, stream, x, xrows, xs, w, dy, bounds, n_docs, T, C, rows, act, dx, dxrows, dxs, part); break;
     default: hipLaunchKernelGGL(conv_bwd_kernel<4>, grid, block, 0, stream, x, xrows, xs, w, dy, bounds, n_docs, T, C, rows, act, dx, dxrows, dxs, part); break;
   }
-  launch_colsum(part, parts, C * K, dw, stream);
 }
 
 // The same sums for few columns (n % 4 == 0) and many parts: a workgroup of 1024 threads
-// takes four float4 columns (64 bytes of a part's row, one quad of lanes) and sums parts
+// takes the four float4 columns from 16 blk on (64 bytes of a part's row, one quad of lanes) and sums parts
 // stripe, stripe + 256, ... in each of 256 stripes (8 loads in flight), then the stripes
 // pairwise (a fixed order).  With one workgroup for all columns, one CU read everything:
 // 2048 parts of 32 columns, or 1024 of 128, took 6.7 us; with a workgroup per 16 columns 4.4.
-__global__ __launch_bounds__(1024) void colsum_narrow_kernel(const float* __restrict__ part, int parts, int n,
-                                                            float* __restrict__ out) {
-  __shared__ f32x4 red[1024];
-  const int n4 = n / 4, c4 = 4 * blockIdx.x + (threadIdx.x & 3), stripe = threadIdx.x >> 2;
+constexpr int SUM_THREADS = 1024;
+__device__ __forceinline__ void narrow_sum(const float* __restrict__ part, int parts, int n, int blk, f32x4* red,
+                                           float* __restrict__ out) {
+  const int n4 = n / 4, c4 = 4 * blk + (threadIdx.x & 3), stripe = threadIdx.x >> 2;
   f32x4 acc = f32x4{};
   if (c4 < n4) {
     const f32x4* p = reinterpret_cast<const f32x4*>(part) + c4;
@@ -362,7 +359,7 @@ __global__ __launch_bounds__(1024) void colsum_narrow_kernel(const float* __rest
   red[threadIdx.x] = acc;
   __syncthreads();
 #pragma unroll
-  for (int half = 512; half >= 4; half >>= 1) {
+  for (int half = SUM_THREADS / 2; half >= 4; half >>= 1) {
     if ((int)threadIdx.x < half) red[threadIdx.x] += red[threadIdx.x + half];
     __syncthreads();
   }
@@ -373,16 +370,68 @@ __global__ __launch_bounds__(1024) void colsum_narrow_kernel(const float* __rest
   }
 }
 
-void launch_colsum(const float* part, int parts, int n, float* out, hipStream_t stream) {
-  if (n <= 256 && parts > 64)
-    hipLaunchKernelGGL(colsum_narrow_kernel, dim3((n + 15) / 16), dim3(1024), 0, stream, part, parts, n, out);
-  else
-    hipLaunchKernelGGL(colsum_kernel<false>, dim3((n / 4 + 63) / 64), dim3(256), 0, stream, part, parts, n, out);
+__global__ __launch_bounds__(SUM_THREADS) void colsum_narrow_kernel(const float* __restrict__ part, int parts, int n,
+                                                                   float* __restrict__ out) {
+  __shared__ f32x4 red[SUM_THREADS];
+  narrow_sum(part, parts, n, blockIdx.x, red, out);
 }
 
-void launch_colsum_add(const float* part, int parts, int n, float* out, hipStream_t stream) {
-  if (parts > 0)
-    hipLaunchKernelGGL(colsum_kernel<true>, dim3((n / 4 + 63) / 64), dim3(256), 0, stream, part, parts, n, out);
+// The parameter gradients of the event inputs in one launch.  Workgroups below `wide` take
+// 256 columns of dw [n]: the conv's parts and, for the q channels (the first nq columns),
+// the query conv's, rows wave, wave + 16, ... in each of 16 waves, then the waves in order.
+// The others take 16 columns each of dgate [ng] (narrow_sum).  A handful of loads per lane,
+// so a launch costs its latency, not its bytes: the three launches before it (the conv's
+// sum, the queries' added to it, the gates') took 4.7, 4.7 and 4.6 us, this one 5.0.
+__global__ __launch_bounds__(SUM_THREADS) void event_sums_kernel(const float* __restrict__ cpart, int cparts, int n,
+                                                                const float* __restrict__ qpart, int qparts, int nq,
+                                                                float* __restrict__ dw, int wide,
+                                                                const float* __restrict__ gpart, int gparts, int ng,
+                                                                float* __restrict__ dgate) {
+  __shared__ f32x4 red[SUM_THREADS];
+  if ((int)blockIdx.x >= wide) {
+    narrow_sum(gpart, gparts, ng, blockIdx.x - wide, red, dgate);
+    return;
+  }
+  constexpr int WAVES = SUM_THREADS / 64, AHEAD = 4;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, j = (blockIdx.x * 64 + lane) * 4;
+  f32x4 acc = f32x4{};
+  // rows past the end re-read the last one and are left out of the sum
+  auto add = [&](const float* part, int parts, int width) {
+    const f32x4* p = reinterpret_cast<const f32x4*>(part + j);
+    const size_t stride = (size_t)width / 4;
+    for (int b = wave; b < parts; b += WAVES * AHEAD) {
+      f32x4 v[AHEAD];
+#pragma unroll
+      for (int q = 0; q < AHEAD; ++q) v[q] = p[(size_t)min(b + WAVES * q, parts - 1) * stride];
+#pragma unroll
+      for (int q = 0; q < AHEAD; ++q)
+        if (b + WAVES * q < parts) acc += v[q];
+    }
+  };
+  if (j < n) add(cpart, cparts, n);
+  if (j < nq) add(qpart, qparts, nq);
+  red[threadIdx.x] = acc;
+  __syncthreads();
+  if (wave == 0 && j < n) {
+#pragma unroll
+    for (int w = 1; w < WAVES; ++w) acc += red[64 * w + lane];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) dw[j + q] = acc[q];
+  }
+}
+
+void launch_colsum(const float* part, int parts, int n, float* out, hipStream_t stream) {
+  if (n <= 256 && parts > 64)
+    hipLaunchKernelGGL(colsum_narrow_kernel, dim3((n + 15) / 16), dim3(SUM_THREADS), 0, stream, part, parts, n, out);
+  else
+    hipLaunchKernelGGL(colsum_kernel, dim3((n / 4 + 63) / 64), dim3(256), 0, stream, part, parts, n, out);
+}
+
+void launch_event_sums(const float* cpart, int cparts, int n, const float* qpart, int qparts, int nq, float* dw,
+                       const float* gpart, int gparts, int ng, float* dgate, hipStream_t stream) {
+  const int wide = (n / 4 + 63) / 64, narrow = (ng + 15) / 16;
+  hipLaunchKernelGGL(event_sums_kernel, dim3(wide + narrow), dim3(SUM_THREADS), 0, stream, cpart, cparts, n, qpart,
+                     qparts, nq, dw, wide, gpart, gparts, ng, dgate);
 }
 
 }  // namespace cqgdn

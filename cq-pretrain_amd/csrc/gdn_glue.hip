@@ -458,12 +458,10 @@ void launch_events_bwd(const EvArgs& a, const EvGrads& d, const int32_t* content
   if (a.n_c > 0) {
     if (d.dcont)  // per-content-row gradients, folded into the hidden rows below
       launch_conv_bwd(a.raw, a.order, a.raw_stride, a.w, w.dconv, content_bounds, n_content_docs, a.n_c, C,
-                      a.K, 1, d.dcont, nullptr, C, d.dw, w.cpart, stream);
+                      a.K, 1, d.dcont, nullptr, C, w.cpart, stream);
     else
       launch_conv_bwd(a.raw, a.order, a.raw_stride, a.w, w.dconv, content_bounds, n_content_docs, a.n_c, C,
-                      a.K, 1, d.draw, a.order, d.draw_stride, d.dw, w.cpart, stream);
-  } else {
-    launch_colsum(w.cpart, 0, C * a.K, d.dw, stream);  // zeros
+                      a.K, 1, d.draw, a.order, d.draw_stride, w.cpart, stream);
   }
   if (a.n_hrows > 0) {
     switch (a.K) {
@@ -474,8 +472,9 @@ void launch_events_bwd(const EvArgs& a, const EvGrads& d, const int32_t* content
   }
   if (d.dcont && d.n_fold > 0)
     hipLaunchKernelGGL(events_bwd_fold_kernel, dim3(d.n_fold), dim3(512), 0, stream, a, d);
-  launch_colsum(w.gpart, a.n_c, 2 * H, d.dgate, stream);
-  launch_colsum_add(w.qpart, qb, SK * a.K, d.dw, stream);  // the query conv's taps: the q channels, first in dw
+  // the query conv's taps are those of the q channels, first in dw
+  launch_event_sums(w.cpart, a.n_c > 0 ? conv_parts(a.n_c) : 0, C * a.K, w.qpart, qb, SK * a.K, d.dw, w.gpart, a.n_c,
+                    2 * H, d.dgate, stream);
 }
 
 // ---------------------------------------------------------------------------

@@ -79,10 +79,12 @@ void launch_conv_fwd(const bf16* x, const int32_t* xrows, int64_t xs, const bf16
                      int n_docs, int T, int C, int K, int act, bf16* y, hipStream_t stream);
 void launch_conv_bwd(const bf16* x, const int32_t* xrows, int64_t xs, const bf16* w, const bf16* dy,
                      const int32_t* bounds, int n_docs, int T, int C, int K, int act, bf16* dx, const int32_t* dxrows,
-                     int64_t dxs, float* dw, float* part, hipStream_t stream);
+                     int64_t dxs, float* part, hipStream_t stream);  // dw parts [conv_parts(T)][C][K], not their sum
 // out[j] = sum over p < parts of part[p][j], fixed order (gdn_conv.hip); n % 4 == 0, 16-byte aligned part
 void launch_colsum(const float* part, int parts, int n, float* out, hipStream_t stream);
-void launch_colsum_add(const float* part, int parts, int n, float* out, hipStream_t stream);  // out += the sums
+// dw[n] = the sum of cpart's rows, plus qpart's in its first nq columns (n, nq % 4 == 0); dgate[ng] = the sum of gpart's
+void launch_event_sums(const float* cpart, int cparts, int n, const float* qpart, int qparts, int nq, float* dw,
+                       const float* gpart, int gparts, int ng, float* dgate, hipStream_t stream);
 // Event inputs of one GatedDelta layer (gdn_glue.hip).  S = H * 128 channels per
 // q/k/v part; index arrays are device int32 (content rows are 0 .. n_c-1, n_c is
 // the zero row / "none").
