@@ -104,7 +104,7 @@ def lib():
 
 
 def ops():
-    """``torch.ops.cqgdn`` (fwd, bwd, recurrent, layer_decode_step), loaded once; raise if unbuilt."""
+    """``torch.ops.cqgdn`` (fwd, bwd, conv1d_fwd, conv1d_bwd, recurrent, layer_decode_step), loaded once; raise if unbuilt."""
     global _OPS
     if _OPS is None:
         lib()  # the operator library links libcqgdn.so: load it (and check it exists) first

@@ -17,6 +17,8 @@
 //       cqgdn_fwd; o is empty with CQGDN_NO_OUTPUT, state empty unless want_state
 //   bwd(q, k, v, g, beta, dy, table, doc, scale, flags, ws?) -> (dq, dk, dv, dg, dbeta)
 //       cqgdn_bwd with the forward's workspace, or cqgdn_bwd_recompute without one
+//   conv1d_fwd(x, weight, bounds, silu) -> y and conv1d_bwd(x, weight, dy, bounds, silu) -> (dx, dweight)
+//       cqgdn_conv1d_fwd / _bwd on [T,C] rows with int32 document bounds; dweight in the weight's dtype
 //   recurrent(q, k, v, g, beta, state!, out!, scale) -> ()
 //       cqgdn_recurrent on [N,t,H,128] (or [t,H,128]) q/k/v/out, value-first fp32 state in place
 //   layer_decode_step(proj, conv_w, A_log, dt_bias, norm_w, conv_history!, state!, heads, key_heads,
@@ -109,6 +111,33 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor, at::Tensor, at::Tensor> bwd(
   return {dq, dk, dv, dg, db};
 }
 
+at::Tensor conv1d_fwd(const at::Tensor& x, const at::Tensor& w, const at::Tensor& bounds, bool silu) {
+  TORCH_CHECK_VALUE(x.dim() == 2 && w.dim() == 2 && w.size(0) == x.size(1), "x must be [T,C] and weight [C,K]");
+  TORCH_CHECK_VALUE(x.scalar_type() == at::kBFloat16 && w.scalar_type() == at::kBFloat16 && x.is_contiguous() &&
+                        w.is_contiguous(),
+                    "x and weight must be contiguous bf16");
+  at::Tensor y = at::empty_like(x);
+  check(cqgdn_conv1d_fwd(cptr(x), cptr(w), bounds.data_ptr<int32_t>(), (int)bounds.numel() - 1, x.size(0),
+                         (int)x.size(1), (int)w.size(1), silu, mptr(y), stream_of(x)),
+        "cqgdn_conv1d_fwd");
+  return y;
+}
+
+std::tuple<at::Tensor, at::Tensor> conv1d_bwd(const at::Tensor& x, const at::Tensor& w, const at::Tensor& dy,
+                                              const at::Tensor& bounds, bool silu) {
+  TORCH_CHECK_VALUE(dy.sizes() == x.sizes() && dy.scalar_type() == at::kBFloat16 && dy.is_contiguous(),
+                    "dy must be contiguous bf16 of x's shape");
+  const int64_t T = x.size(0);
+  const int C = (int)x.size(1), K = (int)w.size(1);
+  at::Tensor dx = at::empty_like(x), dw = at::empty({C, K}, x.options().dtype(at::kFloat));
+  if (T == 0) dw.zero_();  // no rows, no launch
+  at::Tensor ws = bytes(cqgdn_conv1d_bwd_workspace_size(T, C, K), x);
+  check(cqgdn_conv1d_bwd(cptr(x), cptr(w), cptr(dy), bounds.data_ptr<int32_t>(), (int)bounds.numel() - 1, T, C, K,
+                         silu, mptr(dx), dw.data_ptr<float>(), ws.data_ptr(), (size_t)ws.numel(), stream_of(x)),
+        "cqgdn_conv1d_bwd");
+  return {dx, dw.to(w.scalar_type())};
+}
+
 bool on_gpu(const at::Tensor& t) { return t.is_cuda(); }
 
 // ops/gated_delta_net.py:314-352: q, k (l2-normalized), v, out [t,H,128] or [N,t,H,128], one dtype (bf16 or
@@ -188,6 +217,8 @@ TORCH_LIBRARY(cqgdn, m) {
         "Tensor? initial_state, bool want_state) -> (Tensor, Tensor, Tensor)");
   m.def("bwd(Tensor q, Tensor k, Tensor v, Tensor g, Tensor beta, Tensor dy, Tensor table, Tensor doc, float scale, "
         "int flags, Tensor? ws) -> (Tensor, Tensor, Tensor, Tensor, Tensor)");
+  m.def("conv1d_fwd(Tensor x, Tensor weight, Tensor bounds, bool silu) -> Tensor");
+  m.def("conv1d_bwd(Tensor x, Tensor weight, Tensor dy, Tensor bounds, bool silu) -> (Tensor, Tensor)");
   m.def("recurrent(Tensor q, Tensor k, Tensor v, Tensor g, Tensor beta, Tensor(a!) state, Tensor(b!) out, "
         "float scale) -> ()");
   m.def("layer_decode_step(Tensor proj, Tensor conv_w, Tensor A_log, Tensor dt_bias, Tensor norm_w, "
@@ -197,6 +228,8 @@ TORCH_LIBRARY(cqgdn, m) {
 TORCH_LIBRARY_IMPL(cqgdn, CUDA, m) {
   m.impl("fwd", &fwd);
   m.impl("bwd", &bwd);
+  m.impl("conv1d_fwd", &conv1d_fwd);
+  m.impl("conv1d_bwd", &conv1d_bwd);
   m.impl("recurrent", &recurrent);
   m.impl("layer_decode_step", &layer_decode_step);
 }
