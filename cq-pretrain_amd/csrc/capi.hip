@@ -74,7 +74,7 @@ std::mutex g_static_mu;
 void* g_static_ws[kMaxDevices] = {};
 
 // The side stream and its two events: cqgdn_bwd_recompute runs the forward scan
-// on it, cqgdn_bwd its bwd_dkw beside the reverse scan.
+// on it or, as cqgdn_bwd, its bwd_dkw beside the reverse scan.
 // One set per (thread, device), created on first use and kept until the process
 // ends.  Per thread, so that a caller capturing a HIP graph never shares them with
 // another thread's calls.
@@ -131,6 +131,30 @@ int side_beside_scan(int64_t T, int H, int64_t n_chunks, int n_docs, ScanSide** 
   ScanSide* side = nullptr;
   if (const int err = scan_side(&side)) return err;
   if ((int64_t)H * 8 * n_docs * 2 <= side->cus) *out = side;
+  return CQGDN_OK;
+}
+
+// The order of cqgdn_bwd_recompute: the rebuilt forward's scan on the side stream (*scan) beside
+// bwd_local and the reverse scan, bwd_dkw beside the reverse scan (*beside), or one kernel after
+// another (both null).  The two scans side by side pay while each workgroup of the forward's has a
+// CU to itself (FWD_ALONE_LDS) and the reverse scan still has as many; sharing CUs, as two scans of
+// many workgroups must, they halve each other.  us a call (one after another / bwd_dkw beside /
+// scans side by side): 4 heads x 144 chunks 229 / 238 / 160, 8 x 512 1024 / 954 / 860, 16 x 36 122 / - /
+// 107, 16 x 100 301 / 281 / 286, 16 x 144 423 / 380 / 412, 16 x 256 742 / 673 / 686, 16 x 512 1577 /
+// 1405 / 1313, 8 x 2 x 256 835 / 727 / 682, 4 x 2 x 320 635 / 596 / 572; with more workgroups 32 x 64
+// 320 / - / 384, 8 x 3 x 64 266 / - / 287.  Documents of few chunks end before the side stream has
+// started: 16 chunks of 4 / 16 heads 61.9 / - / 58.3, 69.9 / - / 64.5, 8 chunks 52 / - / 51.5, 55.9 /
+// - / 55, 5 chunks 47.7 / - / 49.5, 1 chunk 42.5 / - / 60 (replayed from a graph 16 chunks are even).
+constexpr int kRecomputeMinChunks = 16, kRecomputeBesideMaxChunkHeads = 4096;
+int recompute_order(int64_t T, int H, int64_t n_chunks, int n_docs, ScanSide** scan, ScanSide** beside) {
+  *scan = *beside = nullptr;
+  if (n_chunks < (int64_t)kRecomputeMinChunks * n_docs) return CQGDN_OK;
+  if (const int err = side_beside_scan(T, H, n_chunks, n_docs, beside)) return err;
+  ScanSide* side = nullptr;
+  if (const int err = scan_side(&side)) return err;
+  const int64_t workgroups = (int64_t)H * 8 * n_docs;
+  if (*beside && (workgroups * 4 <= side->cus || n_chunks * H > kRecomputeBesideMaxChunkHeads)) *beside = nullptr;
+  if (!*beside && workgroups * 2 <= side->cus) *scan = side;
   return CQGDN_OK;
 }
 
@@ -407,16 +431,17 @@ int cqgdn_bwd_recompute(const void* q, const void* k, const void* v, const float
                              dbeta, stream, false, nullptr))
     return e;
   if (T == 0) return ok();
-  ScanSide* side = nullptr;
-  if (const int e = scan_side(&side)) return e;
+  ScanSide *scan = nullptr, *beside = nullptr;
+  if (const int e = recompute_order(T, H, n_chunks, n_docs, &scan, &beside)) return e;
   const unsigned fflags = (flags & (CQGDN_NORMALIZE | CQGDN_FP16)) | CQGDN_TRAINING | CQGDN_NO_OUTPUT;
   if (const int e = fwd_impl(q, k, v, g, beta, T, H, chunk_table, n_chunks, doc_chunk, n_docs, scale, fflags, nullptr,
-                             nullptr, nullptr, fwd_workspace, fwd_workspace_bytes, stream, side->stream, side->fork,
-                             side->join))
+                             nullptr, nullptr, fwd_workspace, fwd_workspace_bytes, stream, scan ? scan->stream : nullptr,
+                             scan ? scan->fork : nullptr, scan ? scan->join : nullptr))
     return e;
   return bwd_impl(q, k, v, g, beta, dout, T, H, chunk_table, n_chunks, doc_chunk, n_docs, scale, flags,
                   fwd_workspace, fwd_workspace_bytes, bwd_workspace, bwd_workspace_bytes, dq, dk, dv, dg, dbeta, stream,
-                  true, side->join);
+                  true, scan ? scan->join : nullptr, beside ? beside->stream : nullptr, beside ? beside->fork : nullptr,
+                  beside ? beside->join : nullptr);
 }
 
 int cqgdn_recurrent(const void* q, const void* k, const void* v, const float* g, const void* beta, int dtype_flags,

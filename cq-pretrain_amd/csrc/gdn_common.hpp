@@ -551,6 +551,8 @@ constexpr int SCAN_THREADS = 256;
 constexpr int SCAN_DEPTH = 4;    // chunks whose operands are in flight or in registers
 constexpr int SCAN_SROW = 136;   // row stride (elements) of the state's [v][k] exchange tile
 constexpr int SCAN_VROW = 72;    // row stride (elements) of the [v][t] exchange tile
+constexpr int SCAN_EXCHANGE_BYTES = 16 * (SCAN_SROW + SCAN_VROW) * 2;  // both tiles
+constexpr int LDS_BYTES = 160 * 1024;  // of a CU
 
 // What a scan needs to know of the chunks it requests: where their event rows are (the
 // rows of head h of an [events][H][128] tensor, as a raw buffer that ends after the

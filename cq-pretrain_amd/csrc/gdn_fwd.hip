@@ -429,6 +429,16 @@ __global__ __launch_bounds__(256, 3) void fwd_prep_kernel(
 // reorder a window's own): a full step issues 11 (9 loads, 2 stores), and the Kg^T loads
 // and the store of h^T of its own step precede the wait.
 constexpr int FWD_STEP_OPS = 11, FWD_LOAD_OPS = 9;
+
+// LDS that a workgroup of a scan on the side stream takes in addition, unused: with it none of
+// the reverse scan (SCAN_EXCHANGE_BYTES), which runs beside it, shares its CU.  On a shared CU
+// the two halve each other: the backward with its forward rebuilt, us, H = 16 / 4 / 8, one document
+// of 144 / 144 / 512 chunks: 482 / 208 / 1134, alone on its CU 412 / 160 / 860 (two loader waves and
+// 136 KB a workgroup, which never shared, 434 / 199 / 924).
+constexpr int FWD_RING_BYTES = SCAN_DEPTH * 64 * D * 2, FWD_ALONE_LDS = 84 * 1024;
+static_assert(FWD_RING_BYTES + SCAN_EXCHANGE_BYTES + FWD_ALONE_LDS + SCAN_EXCHANGE_BYTES > LDS_BYTES &&
+                  FWD_RING_BYTES + SCAN_EXCHANGE_BYTES + FWD_ALONE_LDS <= LDS_BYTES,
+              "one forward scan workgroup fits a CU, a reverse scan workgroup no longer");
 template <class E>
 __global__ __launch_bounds__(SCAN_THREADS, 2) void fwd_scan_kernel(
     // without __restrict__ where loads are requested ahead: the barriers then pin their place
@@ -820,7 +830,7 @@ static hipError_t launch_fwd_t(const FwdArgs& a, float* vscale, int vs_target, h
   }
   {
     TimedLaunch tl(K_FWD_SCAN, ss);
-    hipLaunchKernelGGL(fwd_scan_kernel<E>, grid_s, dim3(SCAN_THREADS), 0, ss, ws[F_W], ws[F_UT], ws[F_KGT], gcum,
+    hipLaunchKernelGGL(fwd_scan_kernel<E>, grid_s, dim3(SCAN_THREADS), a.scan_stream ? FWD_ALONE_LDS : 0, ss, ws[F_W], ws[F_UT], ws[F_KGT], gcum,
                        a.chunks, a.doc_chunk, a.H, vscale, a.initial_state, a.final_state, ws[F_HT], ws[F_VNT]);
   }
   if (a.scan_stream)

@@ -29,7 +29,8 @@ struct FwdArgs {
   uint8_t* ws;
   size_t off[F_COUNT];
   // optional: the state scan runs on scan_stream, after scan_fork (recorded on the
-  // caller's stream behind fwd_prep); scan_join is recorded behind it
+  // caller's stream behind fwd_prep), each workgroup with a CU to itself; scan_join is
+  // recorded behind it
   hipStream_t scan_stream;
   hipEvent_t scan_fork, scan_join;
 };

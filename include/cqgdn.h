@@ -165,11 +165,13 @@ int cqgdn_bwd(const void* q, const void* k, const void* v, const float* g, const
  * were kept (ops/gated_delta_net.py:188-194: recompute_w_u_fwd and
  * chunk_gated_delta_rule_fwd_h, then the chain of :195-214).  Arguments as cqgdn_fwd and
  * cqgdn_bwd; fwd_workspace is written here and needs no contents on entry.
- * The rebuilt forward state scan runs on a second stream beside the backward's local
- * kernel and reverse scan (neither reads h or v_new; each scan holds half of the CUs),
- * and the last backward kernel waits for it.  That stream and its two events are
- * created on a thread's first call on a device and kept until the process ends; the
- * call orders them against `stream` with events, so it can be captured in a HIP graph.
+ * Where the scans have few workgroups (one per head, 16-wide value slice and document, on
+ * at most half of the CUs) and the documents are not short, the rebuilt forward scan runs on a
+ * second stream beside the backward's local kernel and reverse scan (neither reads h or v_new),
+ * or the last backward kernel beside the reverse scan as in cqgdn_bwd; otherwise one kernel
+ * runs after another.  That stream and its two events are created on a thread's first such call
+ * on a device and kept until the process ends; the call orders them against `stream` with
+ * events, so it can be captured in a HIP graph.
  */
 int cqgdn_bwd_recompute(const void* q, const void* k, const void* v, const float* g, const float* beta,
                         const void* dout, int64_t T, int H, const int32_t* chunk_table, int64_t n_chunks,

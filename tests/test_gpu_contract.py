@@ -425,10 +425,10 @@ def test_fused_mode_matches_cached_mode(gdn, monkeypatch):
 
 
 def test_fused_mode_matches_cached_mode_at_config2_size(gdn, monkeypatch):
-    """At config 2's size (T = 9216, H = 16) the fused backward's rebuilt state scan runs beside its
-    local kernel and reverse scan for about 100 us; the last kernel must see its h and v_new, so every
-    gradient equals the cached mode's bitwise (the cached mode is checked against the oracle at this
-    size in test_gpu_parity.py)."""
+    """At config 2's size (T = 9216, H = 16) the fused backward rebuilds the workspace and then runs as
+    the cached one, bwd_dkw beside the reverse scan (the other orders are in
+    test_gpu_recompute_order.py): every gradient equals the cached mode's bitwise (the cached mode is
+    checked against the oracle at this size in test_gpu_parity.py)."""
     from cqgdn import synthetic
 
     T, mask, bounds = synthetic.config_events(2, seed=0)
