@@ -334,7 +334,10 @@ __global__ __launch_bounds__(SCAN_THREADS, 2) void bwd_scan_kernel(
   // per-lane parts of the addresses, the same for every chunk (bytes of global memory;
   // elements of LDS)
   const int q = (lane >> 2) & 3, p = lane & 3, from = tile_source(lane);
-  const int f_off = 4096 * wave + 16 * lane;                        // fragments (wave, j) of Kn, (wave, m, b) of -W^T
+  const int f_off = 4096 * wave + 16 * lane;                        // fragments (wave, m, b) of -W^T
+  int n_off[4];                                                     // fragments (wave, j) of Kn, this wave's own k first
+#pragma unroll
+  for (int j = 0; j < 4; ++j) n_off[j] = f_off + 1024 * ((wave + j) & 3);
   const int l_off = (4 * q4 + q) * CH * 2 + 32 * wave + 8 * p;      // dv_local^T row 4 q4 + q, t = 16 wave + 4 p ..
   const int x_off = (4 * q4 + q) * D * 2 + 64 * wave + 16 * p;      // X^T row 4 q4 + q, k = 32 wave + 8 p ..
   const int s_own = r * SCAN_SROW + 32 * wave + 8 * q4;
@@ -348,7 +351,7 @@ __global__ __launch_bounds__(SCAN_THREADS, 2) void bwd_scan_kernel(
   // l: the step's place after the table's and the blocks' first
   auto issue_n = [&](int slot, int l) __attribute__((always_inline)) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) fn[slot][j] = buf_ld16<X8>(kb.buffer(), f_off, kb.offset(l) + 1024 * ((wave + j) & 3));
+    for (int j = 0; j < 4; ++j) fn[slot][j] = buf_ld16<X8>(kb.buffer(), n_off[j], kb.offset(l));
     fl[slot] = buf_ld8<X4>(lb.buffer(), l_off, lb.offset(l));
     fx[slot] = buf_ld16<X8>(xb.buffer(), x_off, xb.offset(l));
     gl[slot] = tab.glast(l);
