@@ -354,7 +354,6 @@ __global__ __launch_bounds__(SCAN_THREADS, 2) void bwd_scan_kernel(
     for (int j = 0; j < 4; ++j) fn[slot][j] = buf_ld16<X8>(kb.buffer(), n_off[j], kb.offset(l));
     fl[slot] = buf_ld8<X4>(lb.buffer(), l_off, lb.offset(l));
     fx[slot] = buf_ld16<X8>(xb.buffer(), x_off, xb.offset(l));
-    gl[slot] = tab.glast(l);
   };
   auto issue_w = [&](int slot, int l) __attribute__((always_inline)) {
 #pragma unroll
@@ -372,6 +371,14 @@ __global__ __launch_bounds__(SCAN_THREADS, 2) void bwd_scan_kernel(
   for (int i = 0; i < SCAN_DEPTH; ++i) {
     issue_n(i, i);
     if (i > 0) issue_w(i - 1, i);
+    if (i == 0) {
+      // the first step's requests go out before the wait for the chunk table (documents of one chunk:
+      // the backward of 512 of them, 16 heads, 1097 -> 1053 us)
+      __builtin_amdgcn_sched_barrier(0);
+      tab.open();
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    gl[i] = tab.glast(i);
   }
   kb.advance();
   wb.advance();
@@ -406,7 +413,10 @@ __global__ __launch_bounds__(SCAN_THREADS, 2) void bwd_scan_kernel(
     constexpr int next = (s + 1) % SCAN_DEPTH;
     g_now = __expf(gl[next]);
     next_inputs(next);
-    if constexpr (decltype(more)::value) issue_n(s, s);
+    if constexpr (decltype(more)::value) {
+      issue_n(s, s);
+      gl[s] = tab.glast(s);
+    }
 #pragma unroll
     for (int m = 0; m < 2; ++m) dS[m] = mfma(fw[s][m][0], b0, dS[m]);
 #pragma unroll

@@ -566,17 +566,19 @@ constexpr int LDS_BYTES = 160 * 1024;  // of a CU
 // last are empty.
 class ScanTable {
  public:
-  // the entries of steps 0 .. SCAN_DEPTH
+  // requests the chunk table's entries; open() waits for them and looks up steps 0 .. SCAN_DEPTH
   __device__ __forceinline__ ScanTable(const int32_t* chunks, const float* gc, const void* rows, int first, int sign,
                                        int n, int H, int h, int lane)
       : chunks_(chunks), gc_(gc + h), rows_(reinterpret_cast<uint64_t>(rows) + (uint64_t)h * D * 2), first_(first),
         sign_(sign), n_(n), H_(H), at_(min(lane, SCAN_DEPTH)) {
-    ChunkInfo now = info(0);
+    now_ = info(0);
     next_ = info(SCAN_DEPTH);
     after_ = info(2 * SCAN_DEPTH);
-    gate_ = gate(now);
+  }
+  __device__ __forceinline__ void open() {
+    gate_ = gate(now_);
     next_gate_ = gate(next_);
-    locate(now, 0);
+    locate(now_, 0);
   }
   // on to the entries of steps x .. x + SCAN_DEPTH
   __device__ __forceinline__ void advance(int x) {
@@ -612,7 +614,7 @@ class ScanTable {
   uint64_t rows_;
   int first_, sign_, n_, H_, at_;
   int lo_, hi_, bytes_;
-  ChunkInfo next_, after_;
+  ChunkInfo now_, next_, after_;
   float gate_, next_gate_;
 };
 

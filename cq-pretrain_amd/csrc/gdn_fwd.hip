@@ -474,6 +474,7 @@ __global__ __launch_bounds__(SCAN_THREADS, 2) void fwd_scan_kernel(
   }
   if (n > 0) {
     ScanTable tab(chunks, gc, W, c_begin, 1, n, H, h, lane);
+    tab.open();
     const size_t cb = (size_t)c_begin * H + h;
     const int64_t tile = (int64_t)H * D * CH * 2;  // bytes from one chunk's [D][64] tile to the next chunk's
     ScanBlocks<false> ub(UT + cb * (D * CH) + v0 * CH, tile, n);
