@@ -296,7 +296,7 @@ constexpr int BESIDE_LDS = 88 * 1024;
 // two stores.  A step's chunk is announced BWD_ANNOUNCE steps later.
 constexpr int BWD_STEP_OPS = 12, BWD_ANNOUNCE = 3;
 
-template <class E, bool SC1>
+template <class E, bool SC1, bool WIDE>
 __global__ __launch_bounds__(SCAN_THREADS, 2) void bwd_scan_kernel(
     // without __restrict__ where loads are requested ahead: the barriers then pin their place
     const E* knP, const float* gc, const E* dvlT, const E* XT, const E* WT, const int32_t* chunks,
@@ -326,11 +326,11 @@ __global__ __launch_bounds__(SCAN_THREADS, 2) void bwd_scan_kernel(
   ScanTable tab(chunks, gc, nullptr, c_last, -1, n, H, h, lane);
   const size_t cb = (size_t)c_last * H + h;
   const int64_t tile = (int64_t)H * D * CH * 2;  // bytes from one chunk's [D][64] tile to the next chunk's
-  ScanBlocks<true> kb(knP + cb * (D * CH), tile, n);
-  ScanBlocks<true> wb(WT + (cb + H) * (D * CH), tile, n + 1);  // one step behind: its first block is step -1's
-  ScanBlocks<true> lb(dvlT + cb * (D * CH) + v0 * CH, tile, n), xb(XT + cb * (D * D) + v0 * D, 2 * tile, n);
-  ScanBlocks<true> sb(dhS + cb * (D * D) + slice * (D * 16), 2 * tile, n);
-  ScanBlocks<true> nb(dVnS + cb * (CH * D) + slice * (CH * 16), tile, n);
+  ScanBlocks<true, WIDE> kb(knP + cb * (D * CH), tile, n);
+  ScanBlocks<true, WIDE> wb(WT + (cb + H) * (D * CH), tile, n + 1);  // one step behind: its first block is step -1's
+  ScanBlocks<true, WIDE> lb(dvlT + cb * (D * CH) + v0 * CH, tile, n), xb(XT + cb * (D * D) + v0 * D, 2 * tile, n);
+  ScanBlocks<true, WIDE> sb(dhS + cb * (D * D) + slice * (D * 16), 2 * tile, n);
+  ScanBlocks<true, WIDE> nb(dVnS + cb * (CH * D) + slice * (CH * 16), tile, n);
   // per-lane parts of the addresses, the same for every chunk (bytes of global memory;
   // elements of LDS)
   const int q = (lane >> 2) & 3, p = lane & 3, from = tile_source(lane);
@@ -351,15 +351,15 @@ __global__ __launch_bounds__(SCAN_THREADS, 2) void bwd_scan_kernel(
   // l: the step's place after the table's and the blocks' first
   auto issue_n = [&](int slot, int l) __attribute__((always_inline)) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) fn[slot][j] = buf_ld16<X8>(kb.buffer(), n_off[j], kb.offset(l));
-    fl[slot] = buf_ld8<X4>(lb.buffer(), l_off, lb.offset(l));
-    fx[slot] = buf_ld16<X8>(xb.buffer(), x_off, xb.offset(l));
+    for (int j = 0; j < 4; ++j) fn[slot][j] = buf_ld16<X8>(kb.buffer(l), n_off[j], kb.offset(l));
+    fl[slot] = buf_ld8<X4>(lb.buffer(l), l_off, lb.offset(l));
+    fx[slot] = buf_ld16<X8>(xb.buffer(l), x_off, xb.offset(l));
   };
   auto issue_w = [&](int slot, int l) __attribute__((always_inline)) {
 #pragma unroll
     for (int m = 0; m < 2; ++m)
 #pragma unroll
-      for (int b = 0; b < 2; ++b) fw[slot][m][b] = buf_ld16<X8>(wb.buffer(), f_off + 2048 * m + 1024 * b, wb.offset(l));
+      for (int b = 0; b < 2; ++b) fw[slot][m][b] = buf_ld16<X8>(wb.buffer(l), f_off + 2048 * m + 1024 * b, wb.offset(l));
   };
   auto next_inputs = [&](int slot) __attribute__((always_inline)) {
     dvl = tile_exchange(fl[slot], from);
@@ -398,7 +398,7 @@ __global__ __launch_bounds__(SCAN_THREADS, 2) void bwd_scan_kernel(
     if constexpr (decltype(more)::value) issue_w((s + SCAN_DEPTH - 1) % SCAN_DEPTH, s);
 #pragma unroll
     for (int j = 1; j < 4; ++j) acc = mfma(fn[s][j], sx[j - 1], acc);
-    buf_st16<OUT>(sb.buffer(), s_out + sb.offset(s), ds_out);
+    buf_st16<OUT>(sb.buffer(s), s_out + sb.offset(s), ds_out);
     // the first two terms of dS_c = exp(G_last) dS_{c+1} + X + (-W^T) dVn
     const f32x8 xf = cvtf8(x);
 #pragma unroll
@@ -421,7 +421,7 @@ __global__ __launch_bounds__(SCAN_THREADS, 2) void bwd_scan_kernel(
     for (int m = 0; m < 2; ++m) dS[m] = mfma(fw[s][m][0], b0, dS[m]);
 #pragma unroll
     for (int m = 0; m < 2; ++m) dS[m] = mfma(fw[s][m][1], b1, dS[m]);
-    buf_st8<OUT>(nb.buffer(), v_out, nb.offset(s), dv_out);
+    buf_st8<OUT>(nb.buffer(s), v_out, nb.offset(s), dv_out);
     own = to8<E>(f32x8{dS[0][0], dS[0][1], dS[0][2], dS[0][3], dS[1][0], dS[1][1], dS[1][2], dS[1][3]});
     st8(Sx + s_own, own);
     if constexpr (SC1 && decltype(more)::value) {
@@ -1246,10 +1246,13 @@ static hipError_t launch_bwd_t(const BwdArgs& a, hipStream_t stream) {
   }
   {
     TimedLaunch tl(K_BWD_SCAN, stream);
-    const auto kernel = beside ? bwd_scan_kernel<E, true> : bwd_scan_kernel<E, false>;
+    // beside, every workgroup is resident at once: far fewer heads than scan_wide's
+    const auto kernel = beside            ? bwd_scan_kernel<E, true, false>
+                        : scan_wide(a.H) ? bwd_scan_kernel<E, false, true>
+                                         : bwd_scan_kernel<E, false, false>;
     hipLaunchKernelGGL(kernel, dim3(a.H * (D / 16), a.n_docs), dim3(SCAN_THREADS), beside ? BESIDE_LDS : 0, stream,
-                       B(B_KNP), Ff(F_GC),
-                       B(B_DVLT), B(B_XT), B(B_WT), a.chunks, a.doc_chunk, a.H, B(B_DH), B(B_DVN), ready, resident);
+                       B(B_KNP), Ff(F_GC), B(B_DVLT), B(B_XT), B(B_WT), a.chunks, a.doc_chunk, a.H, B(B_DH), B(B_DVN),
+                       ready, resident);
   }
   if (beside) {
     launch_resident_gate(resident, a.H * (D / 16) * a.n_docs, a.side);

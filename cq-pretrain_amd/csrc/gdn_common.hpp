@@ -621,18 +621,24 @@ class ScanTable {
 // One head's block of a [chunks][H][..] buffer over the steps of a scan (REVERSE: from
 // the last chunk down): a round's chunks are reached from one raw buffer with the
 // step's place in the round as a scalar offset, so a step computes no address.  Steps
-// past the last lie past the buffer's end: loads return zeros.
-template <bool REVERSE>
+// past the last lie past the buffer's end: loads return zeros.  A raw buffer's size and
+// offsets are unsigned 32-bit numbers, enough for a round of the largest buffers (h, X
+// and dS, 32 KB a chunk-head) up to 26,214 heads; for more (WIDE, chosen by scan_wide) every
+// step has a raw buffer of its own, the block up to the next chunk's.
+template <bool REVERSE, bool WIDE>
 class ScanBlocks {
  public:
   // first: the block of step 0; size: bytes from a chunk's block to the next chunk's; n: steps
   __device__ __forceinline__ ScanBlocks(const void* first, int64_t size, int n)
       : at_(reinterpret_cast<uint64_t>(first) - (REVERSE ? SCAN_DEPTH * size : 0)), size_(size), left_(n) {}
-  __device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer() const {
-    return buf_rsrc(reinterpret_cast<const void*>(at_), (SCAN_DEPTH + 1) * (int)size_);
+  __device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer(int l) const {
+    if constexpr (WIDE)
+      return buf_rsrc(reinterpret_cast<const void*>(at_ + place(l) * size_), l < left_ ? (int)(uint32_t)size_ : 0);
+    else
+      return buf_rsrc(reinterpret_cast<const void*>(at_), (int)((SCAN_DEPTH + 1) * (uint32_t)size_));
   }
   __device__ __forceinline__ int offset(int l) const {
-    return (l < left_ ? (REVERSE ? SCAN_DEPTH - l : l) : SCAN_DEPTH + 1) * (int)size_;
+    return WIDE ? 0 : (int)((l < left_ ? place(l) : SCAN_DEPTH + 1) * (uint32_t)size_);
   }
   __device__ __forceinline__ void advance() {
     at_ += (REVERSE ? -SCAN_DEPTH : SCAN_DEPTH) * size_;
@@ -640,10 +646,12 @@ class ScanBlocks {
   }
 
  private:
+  static __device__ __forceinline__ int place(int l) { return REVERSE ? SCAN_DEPTH - l : l; }
   uint64_t at_;
   int64_t size_;
   int left_;
 };
+inline bool scan_wide(int H) { return (uint64_t)(SCAN_DEPTH + 1) * H * (D * D * 2) > UINT32_MAX; }
 
 // a number as a type, for the scans' unrolled steps
 template <int N>

@@ -439,7 +439,7 @@ constexpr int FWD_RING_BYTES = SCAN_DEPTH * 64 * D * 2, FWD_ALONE_LDS = 84 * 102
 static_assert(FWD_RING_BYTES + SCAN_EXCHANGE_BYTES + FWD_ALONE_LDS + SCAN_EXCHANGE_BYTES > LDS_BYTES &&
                   FWD_RING_BYTES + SCAN_EXCHANGE_BYTES + FWD_ALONE_LDS <= LDS_BYTES,
               "one forward scan workgroup fits a CU, a reverse scan workgroup no longer");
-template <class E>
+template <class E, bool WIDE>
 __global__ __launch_bounds__(SCAN_THREADS, 2) void fwd_scan_kernel(
     // without __restrict__ where loads are requested ahead: the barriers then pin their place
     const E* W, const E* UT, const E* KgT, const float* gc, const int32_t* chunks,
@@ -477,9 +477,9 @@ __global__ __launch_bounds__(SCAN_THREADS, 2) void fwd_scan_kernel(
     tab.open();
     const size_t cb = (size_t)c_begin * H + h;
     const int64_t tile = (int64_t)H * D * CH * 2;  // bytes from one chunk's [D][64] tile to the next chunk's
-    ScanBlocks<false> ub(UT + cb * (D * CH) + v0 * CH, tile, n);
-    ScanBlocks<false> kb(KgT + (cb - H) * (D * CH), tile, n + 1);  // one step behind: its first block is step -1's
-    ScanBlocks<false> vb(vnT + cb * (D * CH) + v0 * CH, tile, n), hb(hT + cb * (D * D) + v0 * D, 2 * tile, n);
+    ScanBlocks<false, WIDE> ub(UT + cb * (D * CH) + v0 * CH, tile, n);
+    ScanBlocks<false, WIDE> kb(KgT + (cb - H) * (D * CH), tile, n + 1);  // one step behind: its first block is step -1's
+    ScanBlocks<false, WIDE> vb(vnT + cb * (D * CH) + v0 * CH, tile, n), hb(hT + cb * (D * D) + v0 * D, 2 * tile, n);
     // per-lane parts of the addresses, the same for every chunk (bytes of global
     // memory; elements of LDS)
     const int q = (lane >> 2) & 3, p = lane & 3, from = tile_source(lane);
@@ -504,7 +504,7 @@ __global__ __launch_bounds__(SCAN_THREADS, 2) void fwd_scan_kernel(
     float gl[SCAN_DEPTH];
     // l: the step's place after the table's and the blocks' first
     auto issue_w = [&](int slot, int l) __attribute__((always_inline)) {
-      const __amdgpu_buffer_rsrc_t wr = tab.rows(l), ur = ub.buffer();
+      const __amdgpu_buffer_rsrc_t wr = tab.rows(l), ur = ub.buffer(l);
 #pragma unroll
       for (int i = 0; i < 4; ++i)
         __builtin_amdgcn_raw_ptr_buffer_load_lds(wr, (lds_void_ptr)(ring[slot] + (16 * wave + 4 * i) * D), 16,
@@ -513,7 +513,7 @@ __global__ __launch_bounds__(SCAN_THREADS, 2) void fwd_scan_kernel(
       gl[slot] = tab.glast(l);
     };
     auto issue_k = [&](int slot, int l) __attribute__((always_inline)) {
-      const __amdgpu_buffer_rsrc_t kr = kb.buffer();
+      const __amdgpu_buffer_rsrc_t kr = kb.buffer(l);
 #pragma unroll
       for (int m = 0; m < 2; ++m)
 #pragma unroll
@@ -553,7 +553,7 @@ __global__ __launch_bounds__(SCAN_THREADS, 2) void fwd_scan_kernel(
       f32x4 acc = cvtf4(u);
 #pragma unroll
       for (int j = 0; j < 4; ++j) acc = mfma(w[j], sx[j], acc);
-      buf_st16<CPOL_NT>(hb.buffer(), h_off + hb.offset(s), h_out);
+      buf_st16<CPOL_NT>(hb.buffer(s), h_off + hb.offset(s), h_out);
 #pragma unroll
       for (int m = 0; m < 2; ++m) S[m] *= g_now;
       *reinterpret_cast<X4*>(Vx + v_own) = to4<E>(acc);
@@ -570,7 +570,7 @@ __global__ __launch_bounds__(SCAN_THREADS, 2) void fwd_scan_kernel(
 #pragma unroll
       for (int m = 0; m < 2; ++m) S[m] = mfma(fk[s][m][1], b1, S[m]);
       if constexpr (decltype(more)::value) issue_w(s, s);
-      buf_st8(vb.buffer(), vn_off, vb.offset(s), v_out);
+      buf_st8(vb.buffer(s), vn_off, vb.offset(s), v_out);
       st8(Sx + s_own, pack_permv<E>(S[0], S[1]));
       lds_barrier();
     };
@@ -831,7 +831,8 @@ static hipError_t launch_fwd_t(const FwdArgs& a, float* vscale, int vs_target, h
   }
   {
     TimedLaunch tl(K_FWD_SCAN, ss);
-    hipLaunchKernelGGL(fwd_scan_kernel<E>, grid_s, dim3(SCAN_THREADS), a.scan_stream ? FWD_ALONE_LDS : 0, ss, ws[F_W], ws[F_UT], ws[F_KGT], gcum,
+    const auto kernel = scan_wide(a.H) ? fwd_scan_kernel<E, true> : fwd_scan_kernel<E, false>;
+    hipLaunchKernelGGL(kernel, grid_s, dim3(SCAN_THREADS), a.scan_stream ? FWD_ALONE_LDS : 0, ss, ws[F_W], ws[F_UT], ws[F_KGT], gcum,
                        a.chunks, a.doc_chunk, a.H, vscale, a.initial_state, a.final_state, ws[F_HT], ws[F_VNT]);
   }
   if (a.scan_stream)
