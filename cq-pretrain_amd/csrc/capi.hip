@@ -511,7 +511,7 @@ int cqgdn_conv1d_fwd(const void* x, const void* weight, const int32_t* bounds, i
 
 size_t cqgdn_conv1d_bwd_workspace_size(int64_t T, int C, int K) {
   if (T <= 0 || C <= 0 || K <= 0) return 0;
-  return (size_t)conv_parts(T) * (size_t)C * (size_t)K * sizeof(float);
+  return (size_t)conv_parts(T, C) * (size_t)C * (size_t)K * sizeof(float);
 }
 
 int cqgdn_conv1d_bwd(const void* x, const void* weight, const void* dy, const int32_t* bounds, int n_docs, int64_t T,
@@ -526,7 +526,7 @@ int cqgdn_conv1d_bwd(const void* x, const void* weight, const void* dy, const in
   launch_conv_bwd(static_cast<const bf16*>(x), nullptr, C, static_cast<const bf16*>(weight),
                   static_cast<const bf16*>(dy), bounds, n_docs, (int)T, C, K, activation != 0, static_cast<bf16*>(dx),
                   nullptr, C, static_cast<float*>(workspace), (hipStream_t)stream);
-  launch_colsum(static_cast<const float*>(workspace), conv_parts(T), C * K, dweight, (hipStream_t)stream);
+  launch_colsum(static_cast<const float*>(workspace), conv_parts(T, C), C * K, dweight, (hipStream_t)stream);
   return check_launch("cqgdn_conv1d_bwd");
 }
 
@@ -667,7 +667,7 @@ EvLayout ev_layout(int n_content, int n_queries, int H, int HK, int K, bool fold
   l.dpre = o; o += align256((size_t)n_queries * SK * sizeof(float));
   l.gpart = o; o += align256((size_t)n_content * 2 * H * sizeof(float));
   l.qpart = o; o += align256((size_t)events_query_blocks(n_queries) * SK * K * sizeof(float));
-  l.cpart = o; o += align256((size_t)(n_content > 0 ? conv_parts(n_content) : 0) * C * K * sizeof(float));
+  l.cpart = o; o += align256((size_t)(n_content > 0 ? conv_parts(n_content, (int)C) : 0) * C * K * sizeof(float));
   l.total = o + 256;
   return l;
 }

@@ -111,9 +111,9 @@ __global__ __launch_bounds__(CONV_THREADS) void conv_fwd_kernel(const bf16* __re
   }
 }
 
-// Backward: a wave streams a strip of rows [s, e) for 64 * CONV_BWD_CH channels, walking u = s - (K-1) .. e + K - 2 in groups of K rows whose x and
-// dy rows are requested while the previous group computes (a gathered x row's index
-// one group before that).  Per row u:
+// Backward: a wave streams a strip of rows [s, e) for 64 * CONV_BWD_CH channels, walking u =
+// s - (K-1) .. e + K - 2 in groups of K rows whose x and dy rows are requested while the previous
+// group computes (a gathered x row's index one group before that).  Per row u:
 //   pre[u] from the last K x rows, dpre[u] = dy[u] * silu'(pre[u]),
 //   dw partials over u in [s, e),
 //   dx[t] = sum_j w[K-1-j] * dpre[t + j] over rows t + j of t's document.
@@ -125,7 +125,8 @@ __global__ __launch_bounds__(CONV_THREADS) void conv_fwd_kernel(const bf16* __re
 // partials in LDS, in strip order, and writes one [C][K] part; colsum_kernel (event_sums_kernel in a layer)
 // sums the parts.  Bound by the memory traffic: 8192 rows of 6144 channels take 65.7 us (58 at a large copy's rate),
 // 2048 rows 23.5; a one-wave workgroup and a part per strip took 69.7 and 25.5.
-constexpr int CONV_STRIPS = 128;  // row strips per 64 * CONV_BWD_CH channels
+constexpr int CONV_STRIPS = 128;  // row strips per 64 * CONV_BWD_CH channels, at least
+constexpr int CONV_MIN_GROUPS = 512;  // workgroups to ask for in all: two per CU
 constexpr int CONV_BWD_WAVES = 4; // strips per workgroup
 constexpr int CONV_BWD_CH = 4;    // channels per thread in the backward
 
@@ -305,10 +306,19 @@ __global__ __launch_bounds__(256) void colsum_kernel(const float* __restrict__ p
   }
 }
 
-int conv_strip_rows(int64_t T) { return (int)std::max<int64_t>(16, (T + CONV_STRIPS - 1) / CONV_STRIPS); }
+// Rows of a strip: 16 at least (2 (K - 1) more are read), else T over the strips.  Where
+// CONV_STRIPS strips in fours make fewer workgroups than CONV_MIN_GROUPS (below 4096 channels) there are
+// as many more strips as make that many: with CONV_STRIPS alone whole CUs had nothing to read
+// (65536 rows of 512 / 1536 / 2048 / 3072 channels 266 / 296 / 299 / 337 us, now 53 / 161 / 190 / 309; 8192 rows 43 / 44 / 45 /
+// 50, now 21 / 31 / 32 / 45; with 256 workgroups 78 / 226 / 299 / 337).
+int conv_strip_rows(int64_t T, int C) {
+  const int blocks = (C + 64 * CONV_BWD_CH - 1) / (64 * CONV_BWD_CH);
+  const int strips = std::max(CONV_STRIPS, (CONV_MIN_GROUPS + blocks - 1) / blocks * CONV_BWD_WAVES);
+  return (int)std::max<int64_t>(16, (T + strips - 1) / strips);
+}
 
-int conv_parts(int64_t T) {
-  const int64_t rows = (int64_t)conv_strip_rows(T) * CONV_BWD_WAVES;
+int conv_parts(int64_t T, int C) {
+  const int64_t rows = (int64_t)conv_strip_rows(T, C) * CONV_BWD_WAVES;
   return (int)((T + rows - 1) / rows);
 }
 
@@ -325,7 +335,7 @@ void launch_conv_fwd(const bf16* x, const int32_t* xrows, int64_t xs, const bf16
 void launch_conv_bwd(const bf16* x, const int32_t* xrows, int64_t xs, const bf16* w, const bf16* dy,
                      const int32_t* bounds, int n_docs, int T, int C, int K, int act, bf16* dx, const int32_t* dxrows,
                      int64_t dxs, float* part, hipStream_t stream) {
-  const int rows = conv_strip_rows(T), parts = conv_parts(T);
+  const int rows = conv_strip_rows(T, C), parts = conv_parts(T, C);
   const dim3 grid(parts, (C / CONV_BWD_CH + 63) / 64), block(64 * CONV_BWD_WAVES);
   switch (K) {
     case 2: hipLaunchKernelGGL(conv_bwd_kernel<2>, grid, block, 0, stream, x, xrows, xs, w, dy, bounds, n_docs, T, C, rows, act, dx, dxrows, dxs, part); break;

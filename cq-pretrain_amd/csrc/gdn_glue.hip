@@ -473,7 +473,7 @@ void launch_events_bwd(const EvArgs& a, const EvGrads& d, const int32_t* content
   if (d.dcont && d.n_fold > 0)
     hipLaunchKernelGGL(events_bwd_fold_kernel, dim3(d.n_fold), dim3(512), 0, stream, a, d);
   // the query conv's taps are those of the q channels, first in dw
-  launch_event_sums(w.cpart, a.n_c > 0 ? conv_parts(a.n_c) : 0, C * a.K, w.qpart, qb, SK * a.K, d.dw, w.gpart, a.n_c,
+  launch_event_sums(w.cpart, a.n_c > 0 ? conv_parts(a.n_c, C) : 0, C * a.K, w.qpart, qb, SK * a.K, d.dw, w.gpart, a.n_c,
                     2 * H, d.dgate, stream);
 }
 

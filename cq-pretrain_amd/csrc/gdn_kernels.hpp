@@ -74,13 +74,13 @@ void launch_recurrent(const void* q, const void* k, const void* v, const float* 
                       bool beta_bf16, bool fp16, float* state, void* out, int N, int E, int H, float scale,
                       hipStream_t stream);
 // packed depthwise causal conv1d (gdn_conv.hip); bounds: int32 [n_docs + 1] on the device
-int conv_parts(int64_t T);  // workgroups along the rows of the conv backward (a dw partial each)
+int conv_parts(int64_t T, int C);  // workgroups along the rows of the conv backward (a dw partial each)
 // x row u is x + (xrows ? xrows[u] : u) * xs; dx row t is dx + (dxrows ? dxrows[t] : t) * dxs; y and dy are [T][C]
 void launch_conv_fwd(const bf16* x, const int32_t* xrows, int64_t xs, const bf16* w, const int32_t* bounds,
                      int n_docs, int T, int C, int K, int act, bf16* y, hipStream_t stream);
 void launch_conv_bwd(const bf16* x, const int32_t* xrows, int64_t xs, const bf16* w, const bf16* dy,
                      const int32_t* bounds, int n_docs, int T, int C, int K, int act, bf16* dx, const int32_t* dxrows,
-                     int64_t dxs, float* part, hipStream_t stream);  // dw parts [conv_parts(T)][C][K], not their sum
+                     int64_t dxs, float* part, hipStream_t stream);  // dw parts [conv_parts(T, C)][C][K], not their sum
 // out[j] = sum over p < parts of part[p][j], fixed order (gdn_conv.hip); n % 4 == 0, 16-byte aligned part
 void launch_colsum(const float* part, int parts, int n, float* out, hipStream_t stream);
 // dw[n] = the sum of cpart's rows, plus qpart's in its first nq columns (n, nq % 4 == 0); dgate[ng] = the sum of gpart's
