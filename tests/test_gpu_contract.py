@@ -481,11 +481,11 @@ def test_bwd_recompute_graph_replay(gdn, T, bounds, H, dtype):
             assert torch.equal(o, e), f"replay {replay}: {name} differs"
 
 
-def _bwd_direct(gdn, xs, bounds, do, beside, monkeypatch):
-    """cqgdn_bwd through the C ABI with its workspace in hand; beside=False sets CQGDN_DKW_BESIDE_SCAN=0."""
+def _bwd_call(gdn, xs, bounds, do):
+    """cqgdn_bwd through the C ABI on buffers held here: (run, outputs, counts); run() enqueues the call,
+    counts() reads the workspace's ready counts [chunks][H] and resident count."""
     from cqgdn import _lib
 
-    monkeypatch.setenv("CQGDN_DKW_BESIDE_SCAN", "1" if beside else "0")
     T, H = xs[0].shape[1], xs[0].shape[2]
     q, k, v, g, b = (x.to(DEV).contiguous() for x in xs)
     do_dev = do.to(DEV)
@@ -493,22 +493,39 @@ def _bwd_direct(gdn, xs, bounds, do, beside, monkeypatch):
     _, table, doc = gdn.device_metadata(bounds, DEV)
     nc = table.shape[0]
     bws = torch.full((_lib.lib().cqgdn_bwd_workspace_size(T, H, nc),), 0x5A, dtype=torch.uint8, device=DEV)
-    dq, dk, dv = (torch.empty_like(v) for _ in range(3))
-    dg, db = torch.empty_like(g), torch.empty_like(b)
+    outs = [torch.empty_like(v) for _ in range(3)] + [torch.empty_like(g), torch.empty_like(b)]
     P = gdn._ptr
     flags = _lib.NORMALIZE | _lib.TRAINING | (_lib.FP16 if q.dtype == torch.float16 else 0)
-    gdn.call("cqgdn_bwd", P(q), P(k), P(v), P(g), P(b), P(do_dev), T, H, P(table), nc, P(doc), len(bounds) - 1,
-             128 ** -0.5, flags, P(ws), ws.numel(), P(bws), bws.numel(), P(dq), P(dk), P(dv), P(dg), P(db),
-             gdn._stream(q.device))
+
+    def run():
+        gdn.call("cqgdn_bwd", P(q), P(k), P(v), P(g), P(b), P(do_dev), T, H, P(table), nc, P(doc), len(bounds) - 1,
+                 128 ** -0.5, flags, P(ws), ws.numel(), P(bws), bws.numel(), *(P(x) for x in outs),
+                 gdn._stream(q.device))
+
+    def counts():
+        sync = view(bws, _lib.bwd_offsets(T, H, nc)["sync"], torch.int32, (nc * H + 1,)).cpu()
+        return sync[:-1].view(nc, H), int(sync[-1])
+
+    return run, outs, counts
+
+
+def _bwd_direct(gdn, xs, bounds, do, beside, monkeypatch):
+    """One cqgdn_bwd with its workspace in hand: (gradients, ready counts, resident count).  beside sets
+    CQGDN_DKW_BESIDE_SCAN to 1 (wherever it fits) or 0 (never), None leaves the library's rule."""
+    if beside is None:
+        monkeypatch.delenv("CQGDN_DKW_BESIDE_SCAN", raising=False)
+    else:
+        monkeypatch.setenv("CQGDN_DKW_BESIDE_SCAN", "1" if beside else "0")
+    run, outs, counts = _bwd_call(gdn, xs, bounds, do)
+    run()
     torch.cuda.synchronize()
-    sync = view(bws, _lib.bwd_offsets(T, H, nc)["sync"], torch.int32, (nc * H + 1,)).cpu()
-    return [x.cpu() for x in (dq, dk, dv, dg, db)], sync[:-1].view(nc, H), int(sync[-1])
+    return [x.cpu() for x in outs], *counts()
 
 
 def _beside(H, n_docs, nc):
-    """Whether the library runs the kernel after a state scan beside it: every scan workgroup (one per
-    head, 16-wide value slice and document, a whole CU each) is resident at once on at most half of the
-    CUs, and documents average at least 64 chunks."""
+    """Whether the kernel after a state scan can run beside it (CQGDN_DKW_BESIDE_SCAN=1): every scan
+    workgroup (one per head, 16-wide value slice and document, a whole CU each) is resident at once on at
+    most half of the CUs, and documents average at least 64 chunks."""
     cus = torch.cuda.get_device_properties(0).multi_processor_count
     return H * 8 * n_docs * 2 <= cus and nc >= 64 * n_docs
 
@@ -615,21 +632,19 @@ def test_bwd_dkw_wait_gives_up_with_nan_not_a_hang(gdn, monkeypatch):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-def test_bwd_beside_scan_graph_replay(gdn, dtype):
+def test_bwd_beside_scan_graph_replay(gdn, dtype, monkeypatch):
     """The cached backward with bwd_dkw beside the reverse scan (second stream, fork and join events,
     the counts zeroed by bwd_local inside the call; with fp16 inputs also the scale of dO) captured in a
-    HIP graph: each replay, with eager work between, equals the eager call bitwise."""
+    HIP graph: each replay, with eager work between, equals the eager call bitwise, and leaves the counts
+    of the path that ran (eight value slices a chunk-head, every scan workgroup resident)."""
     T, bounds, H = 4200, (0, 4200), 16
     print(f"case cached bwd beside the scan, graph replay T={T} H={H} {dtype}", flush=True)
-    q, k, v, g, b = (x.to(DEV).contiguous() for x in inputs(T, H, seed=4343))
-    q, k, v = (x.to(dtype) for x in (q, k, v))
-    dy = torch.randn(1, T, H, 128, generator=torch.Generator().manual_seed(4344)).to(dtype).to(DEV)
-    _, _, ws = gdn._forward(q, k, v, g, b, bounds, True, 128 ** -0.5, training=True)
-
-    def run():
-        return gdn._backward(q, k, v, g, b, ws, dy, bounds, True, 128 ** -0.5)
-
-    eager = [x.clone() for x in run()]
+    monkeypatch.setenv("CQGDN_DKW_BESIDE_SCAN", "1")
+    xs = [x.to(dtype) if x.dim() == 4 else x for x in inputs(T, H, seed=4343)]
+    dy = torch.randn(1, T, H, 128, generator=torch.Generator().manual_seed(4344)).to(dtype)
+    run, outs, counts = _bwd_call(gdn, xs, bounds, dy)
+    run()
+    eager = [x.clone() for x in outs]
     torch.cuda.synchronize()
     side = torch.cuda.Stream()
     side.wait_stream(torch.cuda.current_stream())
@@ -638,7 +653,7 @@ def test_bwd_beside_scan_graph_replay(gdn, dtype):
     torch.cuda.current_stream().wait_stream(side)
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.graph(graph):
-        outs = run()
+        run()
     for replay in range(4):
         for o in outs:
             o.fill_(0)
@@ -647,6 +662,8 @@ def test_bwd_beside_scan_graph_replay(gdn, dtype):
         torch.cuda.synchronize()
         for name, o, e in zip(("dq", "dk", "dv", "dg", "dbeta"), outs, eager):
             assert torch.equal(o, e), f"replay {replay}: {name} differs"
+        ready, resident = counts()
+        assert bool((ready == 8).all()) and resident == H * 8, (replay, ready.unique(), resident)
 
 
 @pytest.mark.parametrize("mode", ["cached", "fused"])
