@@ -110,27 +110,32 @@ int scan_side(ScanSide** out) {
   return CQGDN_OK;
 }
 
-constexpr int kBesideMinChunks = 64, kBesideMinChunkHeads = 1280;
+constexpr int kBesideMinChunks = 64, kBesideMinChunkHeads = 1400, kBesideMinWorkgroups = 64;
 
 // The side stream for bwd_dkw beside the reverse scan, or null (*out) when bwd_dkw runs
 // after it.  Each scan workgroup (one per head, 16-wide value slice and document) then has
 // a CU to itself, and bwd_dkw waits for the scan's chunks, so every scan workgroup must be
 // resident at once, leaving at least half of the CUs to bwd_dkw, and the documents must
 // average kBesideMinChunks chunks (below, the side stream's launches and events cost more
-// than the scan takes).  Of those calls it pays where bwd_dkw is long enough: beside / after
-// the scan, us a step: 576 chunk-heads (4 heads x 144) 257 / 248, 1152 (8 x 144) 316 / 315
-// and (8 x 2 x 72) 247 / 244, 1088 (16 x 68) 233 / 236, 2304 (16 x 144) 426 / 452, 4096
-// (8 x 512) 1028 / 1100.  CQGDN_DKW_BESIDE_SCAN in the environment: "0" keeps bwd_dkw after
-// the scan, "1" runs it beside wherever it fits.
+// than the scan takes).  Of those calls it pays where bwd_dkw is long enough and not paced by
+// a scan that is slower beside it.  Beside / after, a step's time, by heads x documents x chunks:
+//   16 x 1 x 66 (1056 chunk-heads) 0.97, x 80 (1280) 1.01, x 90 (1440) 0.99, x 100 0.96, x 144 0.93;
+//   8 x 1 x 140 (1120) 1.01, x 160 (1280) 1.03, x 200 (1600) 0.98, x 320 0.98, x 512 0.95;
+//   8 x 2 x 80 (1280) 1.01, x 100 (1600) 0.93, x 128 0.94; 4 x 4 x 80 (1280) 1.03, x 128 (2048) 0.97;
+//   4 x 2 x 200 (1600) 0.99, x 400 0.92; 4 x 1 (32 workgroups) x 280 / 400 / 640 1.06, x 1024 0.99.
+// CQGDN_DKW_BESIDE_SCAN in the environment: "0" keeps bwd_dkw after the scan, "1" runs it
+// beside wherever it fits.
 int side_beside_scan(int64_t T, int H, int64_t n_chunks, int n_docs, ScanSide** out) {
   *out = nullptr;
   const char* e = getenv("CQGDN_DKW_BESIDE_SCAN");
   if ((e && e[0] == '0') || T <= 0 || H <= 0 || n_docs <= 0) return CQGDN_OK;
   if (n_chunks < (int64_t)kBesideMinChunks * n_docs) return CQGDN_OK;
-  if (!(e && e[0] == '1') && n_chunks * H < kBesideMinChunkHeads) return CQGDN_OK;
+  const int64_t workgroups = (int64_t)H * 8 * n_docs;
+  if (!(e && e[0] == '1') && (n_chunks * H < kBesideMinChunkHeads || workgroups < kBesideMinWorkgroups))
+    return CQGDN_OK;
   ScanSide* side = nullptr;
   if (const int err = scan_side(&side)) return err;
-  if ((int64_t)H * 8 * n_docs * 2 <= side->cus) *out = side;
+  if (workgroups * 2 <= side->cus) *out = side;
   return CQGDN_OK;
 }
 

@@ -631,6 +631,22 @@ def test_bwd_dkw_wait_gives_up_with_nan_not_a_hang(gdn, monkeypatch):
         assert bool(torch.isnan(x.float()).all()), name
 
 
+@pytest.mark.parametrize("H,chunks,beside", [
+    (16, 80, False), (16, 100, True),   # below and above 1400 chunk-heads
+    (4, 400, False), (8, 200, True),    # fewer than 64 scan workgroups; as many
+])
+def test_bwd_dkw_beside_scan_where_it_pays(gdn, H, chunks, beside, monkeypatch):
+    """The library's own rule, by the workspace's counts: bwd_dkw beside the reverse scan announces
+    every chunk-head and every scan workgroup, after it none."""
+    T = 64 * chunks
+    print(f"case bwd_dkw beside by rule: H={H} chunks={chunks}", flush=True)
+    xs = inputs(T, H, seed=27)
+    do = torch.randn(1, T, H, 128, generator=torch.Generator().manual_seed(28)).bfloat16()
+    _, ready, resident = _bwd_direct(gdn, xs, (0, T), do, None, monkeypatch)
+    assert bool((ready == (8 if beside else 0)).all()), ready.unique()
+    assert resident == (H * 8 if beside else 0)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_bwd_beside_scan_graph_replay(gdn, dtype, monkeypatch):
     """The cached backward with bwd_dkw beside the reverse scan (second stream, fork and join events,
