@@ -1,134 +1,122 @@
 """The reverse scan's hand-off to a bwd_dkw running beside it (csrc/gdn_bwd.hip: bwd_scan_kernel's
-loader 1, bwd_dkw_kernel's wait), checked on a model of loader 1's vector-memory queue on the CPU.
+announcements, bwd_dkw_kernel's wait), on a model of the four waves' vector memory queues and on the
+built kernel.
 
-Loader 1 of each value-slice workgroup stores every step's dS / dVn (six stores, the copy-out of
-step tau-1 at iteration tau) and refills its stage part (18 copies, the part of step tau+3).  A
-wave's loads and stores retire in issue order, and it can only wait until at most N of its
-operations are in flight, so N must count exactly the operations it issued after the part it waits
-for.  Beside a bwd_dkw, loader 1 also announces step tau-3's chunk right after its wait at
-iteration tau (one atomic add, in flight with the rest): that wait covers the copy-out of step
-tau-3, and the atomic is itself one more operation the next wait must count.  After the loop it
-stores the last step, waits for everything and announces the steps the loop did not.
+Each wave of a value-slice workgroup stores a quarter of every step's dS and dVn.  A chunk is announced
+(one atomic add, by wave 0) three steps later: at the end of a full step every wave waits until at most 36
+of its operations are in flight, a barrier follows, and wave 0 announces.  A wave's operations retire in
+issue order, so the wait covers a store once at least 36 operations were surely issued after it; the
+compiler keeps an operation inside its window between two barriers and may reorder there, so what counts
+is the operations of whole windows.  After the last step every wave waits for everything, and wave 0
+announces the rest.
 
-The model replays the kernel's loop and its wait counts against a queue in which exactly the last N
-operations are still in flight, and asserts: every wait covers the part it waits for; every
-announcement comes after all six stores of its step have retired; every step is announced exactly
-once, in the order the scan finishes them (so bwd_dkw, which waits for the count of its chunk to
-reach 8, one per value slice, reads a chunk only after every slice's stores of it are visible).  A
-count that assumes an announcement that was not issued, or forgets the copy-out, must fail.
+The model asserts that every announcement follows all stores of its step by all four waves, and that every
+step is announced once, in the order in which the scan finishes them; a looser wait, an announcement a step
+early and one without the barrier must fail.  The built kernel must have the model's operations in its
+windows.
 """
 
 import pytest
 
-PART = 18  # BWD_PART_COPIES[1]
-STORES = 6  # BWD_OUT_STORES
-DEPTH = 3  # BS_DEPTH
+from kernel_windows import LIB, OBJDUMP, windows
+
+DEPTH = 4
+FIRST = 5    # -W^T's four loads and the store of dS, up to the barrier between the contractions
+SECOND = 7   # kdec Kn's four loads, dv_local, X and the store of dVn
+ANNOUNCE = 3
+LIMIT = ANNOUNCE * (FIRST + SECOND)  # BWD_ANNOUNCE * BWD_STEP_OPS
 
 
 class ProtocolError(AssertionError):
     pass
 
 
-def kernel_wait_count(tau, n, announce):
-    """The kernel's vmcnt for loader 1 at iteration tau (bwd_scan_kernel, j == 1)."""
-    xn = tau + 1
-    later = xn + 1 < n
-    stored = tau >= 2
-    announced = announce and tau >= 4
-    if later and announced:
-        return PART + STORES + 1
-    if later and stored:
-        return PART + STORES
-    if later:
-        return PART
-    if announced:
-        return STORES + 1
-    if stored:
-        return STORES
-    return 0
-
-
-def replay(n, announce=True, wait_count=kernel_wait_count):
-    """Loader 1's operations for a document of n chunks; returns the steps announced, in order."""
-    ops = []  # issue order: (kind, step)
+def replay(n, limit=LIMIT, announce=ANNOUNCE, barrier=True):
+    """The steps of a document of n chunks announced, in order."""
+    issued = []  # per window: (step, operations); every wave issues the same
+    known = [0]  # windows surely retired when wave 0 announces, for the wave that knows least
     announced = []
 
-    def retired_upto(inflight):
-        return len(ops) - min(inflight, len(ops))
+    def retired(operations_left):
+        """Windows whose every operation has retired once at most that many are in flight."""
+        left = 0
+        for i in range(len(issued) - 1, -1, -1):
+            if left >= operations_left:
+                return i + 1
+            left += issued[i][1]
+        return 0
 
-    def check_retired(kind, step, upto, what):
-        idx = [i for i, op in enumerate(ops) if op == (kind, step)]
-        if not idx or max(idx) >= upto:
-            raise ProtocolError(f"{what}: {kind} of step {step} may still be in flight")
+    def publish(step):
+        last = max(i for i, (s, _) in enumerate(issued) if s == step)
+        if last >= known[0]:
+            raise ProtocolError(f"step {step} announced while its stores may be in flight")
+        announced.append(step)
 
-    for tau in range(-DEPTH, n):
-        xn, xo, xi = tau + 1, tau - 1, tau + DEPTH
-        if 0 <= xn < n:
-            upto = retired_upto(wait_count(tau, n, announce))
-            check_retired("part", xn, upto, f"iteration {tau}")
-            if announce and tau >= 3:
-                check_retired("store", tau - 3, upto, f"announcing step {tau - 3}")
-                ops.append(("announce", tau - 3))
-                announced.append(tau - 3)
-        if xo >= 0:
-            ops.extend([("store", xo)] * STORES)
-        if xi < n:
-            ops.extend([("part", xi)] * PART)
-    if n > 0:
-        ops.extend([("store", n - 1)] * STORES)
-        if announce:
-            upto = retired_upto(0)  # wait_vmem_all
-            for s in range(max(n - 4, 0), n):
-                check_retired("store", s, upto, f"announcing step {s} after the loop")
-                ops.append(("announce", s))
-                announced.append(s)
+    tau = 0
+    while tau + DEPTH <= n:
+        for _ in range(DEPTH):
+            issued += [(tau, FIRST), (tau, SECOND)]
+            now = retired(limit)
+            if barrier:
+                known[0] = now
+            if tau >= announce:
+                publish(tau - announce)
+            known[0] = now  # without the barrier the other waves are a step behind wave 0
+            tau += 1
+    for _ in range(n - tau):
+        issued += [(tau, 1), (tau, 1)]  # the stores alone
+        tau += 1
+    known[0] = len(issued)
+    for step in range(len(announced), n):
+        publish(step)
     return announced
 
 
-@pytest.mark.parametrize("n", [0, 1, 2, 3, 4, 5, 6, 7, 8, 13, 144])
-@pytest.mark.parametrize("announce", [False, True])
-def test_reverse_scan_announcements_follow_their_stores(n, announce):
-    got = replay(n, announce)
-    if announce:
-        assert sorted(got) == list(range(n)) and len(set(got)) == n
-        # steps are announced in the order they finish: bwd_dkw takes chunks last to first
-        assert got == sorted(got)
-    else:
-        assert got == []
+@pytest.mark.parametrize("n", list(range(14)) + [144])
+def test_reverse_scan_announcements_follow_their_stores(n):
+    assert replay(n) == list(range(n))
 
 
-def test_counting_an_announcement_not_yet_issued_is_caught():
-    def loose(tau, n, announce):
-        xn = tau + 1
-        later, stored = xn + 1 < n, tau >= 2
-        announced = announce and tau >= 3  # one iteration early: that atomic was never issued
-        return (PART if later else 0) + (STORES if stored else 0) + (1 if announced else 0)
-
-    with pytest.raises(ProtocolError, match="may still be in flight"):
-        replay(9, True, loose)
+def test_a_looser_wait_is_caught():
+    with pytest.raises(ProtocolError, match="may be in flight"):
+        replay(9, limit=LIMIT + 1)
 
 
-def test_forgetting_the_announcement_is_safe_but_forgetting_the_copy_out_is_caught():
-    def strict(tau, n, announce):  # one operation fewer in flight than issued: waits longer, still correct
-        return max(kernel_wait_count(tau, n, announce) - (1 if announce and tau >= 4 else 0), 0)
+def test_an_announcement_a_step_early_is_caught():
+    with pytest.raises(ProtocolError, match="may be in flight"):
+        replay(9, announce=ANNOUNCE - 1)
 
-    assert replay(9, True, strict) == list(range(9))
 
-    def loose(tau, n, announce):
-        return kernel_wait_count(tau, n, announce) + (STORES if tau < 2 else 0)
-
-    with pytest.raises(ProtocolError, match="may still be in flight"):
-        replay(9, True, loose)
+def test_an_announcement_without_the_barrier_is_caught():
+    with pytest.raises(ProtocolError, match="may be in flight"):
+        replay(9, barrier=False)
 
 
 def test_chunk_counts_reach_eight_only_after_every_slice():
-    """Eight value slices announce their steps; a chunk's count (chunk = c_end - 1 - step) reaches 8,
+    """Eight value slices announce their steps; a chunk's count (chunk = last - step) reaches 8,
     bwd_dkw's condition, only once every slice has announced that step, each after its own stores."""
     n = 11
     counts = [0] * n
-    per_slice = [replay(n) for _ in range(8)]
-    for s in range(8):
-        for step in per_slice[s]:
+    for done, steps in enumerate(replay(n) for _ in range(8)):
+        assert max(counts) <= done
+        for step in steps:
             counts[n - 1 - step] += 1
     assert counts == [8] * n
 
+
+@pytest.mark.skipif(not (LIB.exists() and OBJDUMP.exists()), reason="needs the built library and llvm-objdump")
+@pytest.mark.parametrize("kernel", ["bwd_scan_kernelIDF16bLb1ELb0EE", "bwd_scan_kernelIDF16_Lb1ELb0EE"])
+def test_the_built_kernel_keeps_its_windows(kernel, tmp_path):
+    ws = windows(kernel, str(tmp_path))
+    full = [i for i, w in enumerate(ws) if i and w.count("load") >= 6 and ws[i - 1].count("load") >= 4
+            and w[-1] == ("wait", LIMIT)]
+    assert len(full) == 2 * DEPTH  # the peeled round, then the loop
+    for i in full:
+        first, second = ws[i - 1], ws[i]
+        assert first.count("load") >= 4 and first.count("store") == 1, first
+        assert second.count("load") >= 6 and second.count("store") == 1, second
+    # announcements: after the barrier behind the wait of the peeled round's last step and of every step of the loop
+    atomics = [i for i, w in enumerate(ws) if i and "atomic" in w]
+    assert [i + 1 for i in full[DEPTH - 1:]] == atomics[:DEPTH + 1]
+    # the rest once nothing is in flight
+    assert ("wait", 0) in [w[-1] for w in ws if w]
