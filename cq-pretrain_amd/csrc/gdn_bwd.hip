@@ -63,7 +63,7 @@ __global__ __launch_bounds__(256, 3) void bwd_local_kernel(
   // grid (H, NC), chunks dispatched first to last: the reverse state scan that
   // follows reads the last chunks first, and they are then the most recently
   // written (still in the memory-side cache).  The scan's other two operands,
-  // the perm32 copy of Kn and -W^T, are made here for the same reason.
+  // kdec Kn and -W^T, are made here for the same reason.
   const HeadChunk hc = xcd_head_chunk(gridDim.x, gridDim.y);  // all heads of a chunk on one XCD
   const int h = hc.h, c = hc.p;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -198,7 +198,7 @@ __global__ __launch_bounds__(256, 3) void bwd_local_kernel(
   }
 
   // dv_local^T (s rows 16 wave + 4 q4 .., 8 value tiles) = P^T dO: P^T comes from
-  // the P tiles (pack_perm, events in perm32 order), dO is read transposed in the
+  // the P tiles (pack_permv, events in perm32 order), dO is read transposed in the
   // same order; only t >= s contributes
   f32x4 dvl[8];
   {
@@ -551,13 +551,13 @@ __global__ __launch_bounds__(256, 2) void bwd_dkw_kernel(
   E* dWs = VnT;                        // dW rows [t][k], from phase 4 on
 
   // This wave's state fragments: rows k = 16 (2 wave + mm) + r of h
-  // (column gathers of h^T) and of dS_{c+1}, value block kb.
+  // (columns of h^T, turned in LDS) and of dS_{c+1}, value block kb.
   const E* ht = hT + cb * (D * D);
   X8 bh[2][4], bd[2][4];
-  // Every prologue load is issued before the first wait: the column gathers'
-  // loads, the gate and k-norm values (unconditional: rk is allocated either
-  // way), the v_new^T rows and the Q, K, dO rows; the gathers' lane exchange
-  // comes last.  The q norm is formed from the Q rows (row_rnorm).
+  // Every prologue load is issued before the first wait: h^T by row pieces, the
+  // gate and k-norm values (unconditional: rk is allocated either way), the
+  // v_new^T rows and the Q, K, dO rows; h^T is turned last.  The q norm is formed
+  // from the Q rows (row_rnorm).
   {
     const int t = tid >> 2, p = tid & 3;
     X8 gh[8];  // h^T row v = 16 i + lane / 4, piece p of the wave's columns k = 32 wave ..
@@ -704,8 +704,8 @@ __global__ __launch_bounds__(256, 2) void bwd_dkw_kernel(
   // ---- phase 2: dQ^T (k-tiles 2w, 2w+1 as rows, t columns); dG_t from the output term ----
   // Each MFMA takes the operands of dQ = dO h^T + (dP Gam) K swapped, so a lane holds 4
   // consecutive k of one row t: dQ[mm][n][i] = dq[t = 16 n + r][k = 16 (2w + mm) + 4 q4 + i].
-  // The row's gate and norm are then one value per lane, its sums over k run over the
-  // 4 lanes of a column (permlane swaps), and dq leaves as 8-byte pieces of rows.
+  // The row's gate and norm are then one value per lane, and its sums over k run over the
+  // 4 lanes of a column (permlane swaps).
   f32x4 dQ[2][4];
   f32x4 qrow[4][2];  // q[t = 16 n + r][k = 16 (2w + mm) + 4 q4 + i], kept for the dq stores
   float pdot[4];     // this wave's parts of the row dots q_t . dQ_t (l2norm backward of dq)
@@ -762,9 +762,9 @@ __global__ __launch_bounds__(256, 2) void bwd_dkw_kernel(
   // The dS fragments (bd) requested after phase 1 have landed long since: wait
   // for them here, where nothing else is in flight, so that their first use in
   // phase 3 does not wait for the dq stores and the dVn copy issued below (the
-  // stores are conditional, so the compiler could only wait for everything).
+  // copy stands in a branch, so the compiler counts the path without it).
   wait_vmem_all();
-  // dq = rq (dQ - q (q . dQ)): each lane stores 4 consecutive k of row t = 16 n + r
+  // dq = rq (dQ - q (q . dQ)): each lane holds 4 consecutive k of row t = 16 n + r
   const int rowb = H * D * 2;  // bytes per event row
   {
   // dq's rows over the dO rows (256-byte rows, 16-byte columns XORed with t % 16), then
@@ -1057,9 +1057,6 @@ __global__ __launch_bounds__(256, 2) void bwd_dkw_kernel(
   }
   lds_barrier();
 
-  // The norms rsn requested in wy phase 1 have landed: wait here, before the
-  // conditional dv stores, so that phase 5 does not wait for those stores.
-  wait_vmem_all();
   // ---- wy phase 4b: dv = beta (T^T dVn) ----
   {
     float colB[4] = {0.f, 0.f, 0.f, 0.f};

@@ -34,7 +34,6 @@ typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x8 __attribute__((ext_vector_type(8)));
 
-__device__ __forceinline__ int lane_id() { return threadIdx.x & 63; }
 
 __device__ __forceinline__ f32x4 mfma(bf16x8 a, bf16x8 b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
@@ -48,12 +47,6 @@ __device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
 
-__device__ __forceinline__ bf16x8 zero8() {
-  bf16x8 z;
-#pragma unroll
-  for (int i = 0; i < 8; ++i) z[i] = (bf16)0.f;
-  return z;
-}
 
 __device__ __forceinline__ bf16x4 cvt4(f32x4 x) { return __builtin_convertvector(x, bf16x4); }
 __device__ __forceinline__ f32x4 cvtf4(bf16x4 x) { return __builtin_convertvector(x, f32x4); }
@@ -102,18 +95,6 @@ __device__ __forceinline__ bf16x8 ld8_tr(const bf16* tile, int ld, int k0, int n
   const i16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(p));
   const i16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(p + 4 * ld));
   return __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-}
-
-// C-layout column from a row-major LDS tile: lane (q4, r) gets tile[row0 + 4 q4 + e][col0 + r],
-// e = 0..3 -- the rows and column an MFMA result fragment holds -- in one ds_read_b64_tr_b16:
-// lane a of each 16-lane group addresses the 4 elements tile[row0 + 4 q4 + (a >> 2)][col0 +
-// 4 (a & 3) ..], and the instruction hands lane j element e of lane (j >> 2) + 4 e, column
-// j & 3 (the layout ld8_tr relies on).  ld and col0 multiples of 4.
-__device__ __forceinline__ bf16x4 ld4_c(const bf16* tile, int ld, int row0, int col0) {
-  typedef __attribute__((address_space(3))) i16x4 lds_i16x4;
-  const int lane = threadIdx.x & 63, r = lane & 15, q4 = lane >> 4;
-  const bf16* p = tile + (row0 + 4 * q4 + (r >> 2)) * ld + col0 + 4 * (r & 3);
-  return __builtin_bit_cast(bf16x4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(p)));
 }
 
 // ---- fp16 operands ----------------------------------------------------------
@@ -192,7 +173,7 @@ __device__ __forceinline__ typename Vec<E>::x8 ld8_trv(const E* tile, int ld, in
 
 // ld8_tr with the rows in perm32 order: lane (q4, r) gets
 // tile[k0 + 4 q4 + e][n0 + r] for e = 0..3 and tile[k0 + 16 + 4 q4 + e - 4][n0 + r]
-// for e = 4..7, the K order of a B (or A) operand built by pack_perm from
+// for e = 4..7, the K order of a B (or A) operand built by pack_permv from
 // accumulator fragments.
 template <class E>
 __device__ __forceinline__ typename Vec<E>::x8 ld8_trpv(const E* tile, int ld, int k0, int n0) {
@@ -280,7 +261,7 @@ __device__ __forceinline__ void columns_from_rows(T* own, typename Vec<T>::x8 x0
   }
 }
 
-// ---- workgroup synchronization for loader/consumer kernels ----------------
+// ---- waits and barriers that leave memory operations in flight ------------
 // Barrier that orders LDS only: waits for this wave's LDS operations, then
 // s_barrier.  __syncthreads() also waits for every outstanding vector-memory
 // operation (including asynchronous global->LDS copies still in flight for
@@ -454,8 +435,8 @@ __device__ __forceinline__ V keep_if(bool in, V x) {
 // A raw buffer resource over the rows of one chunk in an [events][H][128] bf16
 // tensor: based at head h of the chunk's first event, it ends after the last
 // valid row, so the hardware's range check drops stores to rows past the chunk's
-// length (no per-lane branch).  A store's address is a per-lane VGPR offset plus a
-// wave-uniform SGPR offset (the row), instead of a 64-bit address per lane.
+// length (no per-lane branch).  A store's address is one per-lane offset (16-byte stores
+// have no scalar one, see buf_st16), instead of a 64-bit address per lane.
 // 0x00020000 is the resource's fourth dword for a raw buffer on gfx9-family parts.
 typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
 template <class E>  // bf16 or fp16 rows
@@ -477,15 +458,6 @@ template <int CPOL = 0, class X8>
 __device__ __forceinline__ void buf_st16(__amdgpu_buffer_rsrc_t rs, int voff, X8 x) {
   __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, x), rs, voff, 0, CPOL);
 }
-__device__ __forceinline__ void buf_st1(__amdgpu_buffer_rsrc_t rs, int voff, int soff, float x) {
-  __builtin_amdgcn_raw_buffer_store_b16(__builtin_bit_cast(unsigned short, (bf16)x), rs, voff, soff, 0);
-}
-// four values rounded to E (bf16 or fp16), 8 bytes
-template <class E = bf16>
-__device__ __forceinline__ void buf_st4(__amdgpu_buffer_rsrc_t rs, int voff, int soff, f32x4 x) {
-  __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, to4<E>(x)), rs, voff, soff, 0);
-}
-
 template <class X8>
 __device__ __forceinline__ X8 buf_ld16(__amdgpu_buffer_rsrc_t rs, int voff, int soff) {
   return __builtin_bit_cast(X8, __builtin_amdgcn_raw_buffer_load_b128(rs, voff, soff, 0));
@@ -557,8 +529,7 @@ constexpr int LDS_BYTES = 160 * 1024;  // of a CU
 // What a scan needs to know of the chunks it requests: where their event rows are (the
 // rows of head h of an [events][H][128] tensor, as a raw buffer that ends after the
 // chunk's last row, so that rows past it read as zeros) and G of their last event.  A
-// round of SCAN_DEPTH steps looks up steps x .. x + SCAN_DEPTH (one more than a round:
-// the first operand is requested a step early), held in lanes 0 .. SCAN_DEPTH, and a
+// round looks up its SCAN_DEPTH steps, held in lanes 0 .. SCAN_DEPTH - 1, and a
 // step's entry is a few v_readlane.  Each round requests the chunk table entries of two
 // rounds on and the gates of the next (whose rows the entries requested a round before
 // give), so no step waits for them, and without a branch, so that the compiler can count
@@ -566,11 +537,11 @@ constexpr int LDS_BYTES = 160 * 1024;  // of a CU
 // last are empty.
 class ScanTable {
  public:
-  // requests the chunk table's entries; open() waits for them and looks up steps 0 .. SCAN_DEPTH
+  // requests the chunk table's entries; open() waits for them and looks up the first round
   __device__ __forceinline__ ScanTable(const int32_t* chunks, const float* gc, const void* rows, int first, int sign,
                                        int n, int H, int h, int lane)
       : chunks_(chunks), gc_(gc + h), rows_(reinterpret_cast<uint64_t>(rows) + (uint64_t)h * D * 2), first_(first),
-        sign_(sign), n_(n), H_(H), at_(min(lane, SCAN_DEPTH)) {
+        sign_(sign), n_(n), H_(H), at_(min(lane, SCAN_DEPTH - 1)) {
     now_ = info(0);
     next_ = info(SCAN_DEPTH);
     after_ = info(2 * SCAN_DEPTH);
@@ -580,7 +551,7 @@ class ScanTable {
     next_gate_ = gate(next_);
     locate(now_, 0);
   }
-  // on to the entries of steps x .. x + SCAN_DEPTH
+  // on to the round of steps x ..
   __device__ __forceinline__ void advance(int x) {
     locate(next_, x);
     gate_ = next_gate_;

@@ -11,7 +11,7 @@
 //
 // Kernels:
 //   fwd_prep   grid (NC, H), 4 waves: l2norm q,k; cumsum g; A via MFMA; the unit
-//              lower-triangular inverse in LDS (fp32); W, W^T, U via MFMA.
+//              lower-triangular inverse in LDS (fp32); W, U via MFMA.
 //   fwd_scan   grid (H * 8 value slices, docs), 4 waves: the serial scan, a 128x16
 //              fp32 state slice held in registers across all chunks of a document.
 //   fwd_out    grid (NC, H), 4 waves: O^T = gam * (h^T Qn^T) + Vn^T P^T, all MFMA.
