@@ -271,8 +271,9 @@ __global__ __launch_bounds__(256, 3) void bwd_local_kernel(
 // so a lane's eight values of dS are consecutive in k: one 16-byte LDS write, and one
 // 16-byte piece of X^T.
 //
-// Measured (H = 16, one document of 144 chunks / 15 documents, 520 chunks): 116.6 -> 92
-// us, 331 -> 290 us; 36 chunks 32.4 -> 24.2; four heads, 144 chunks 113.6 -> 77.9.
+// Measured in the kernel trace of whole steps, bwd_dkw after it (H = 16, one document of 144
+// chunks / 15 documents, 520 chunks): 121 -> 97 us, 326 -> 298 us; 36 chunks 32.9 -> 23.7;
+// four heads, 144 chunks 113.5 -> 77.1.
 //
 // The outputs are stored with the non-temporal hint: the scan still has the earlier chunks'
 // operands to read (bwd_local wrote them first to last, so they are the oldest in the
@@ -490,8 +491,8 @@ __global__ __launch_bounds__(SCAN_THREADS, 2) void bwd_scan_kernel(
 // leave as whole rows, dq through the dO rows' place before the dVn copy, dk and dv from
 // the K and V rows' places, whose values only their lane still reads: column gathers and
 // 8-byte stores from lanes on 16 different rows keep the vector memory unit 3 and 2.5
-// times as long.  H = 16, 144 chunks / 520 chunks of 15 documents / 36 chunks: 127.5 ->
-// 122.4 / 420 -> 402 / 42.5 -> 40.8 us (the stores alone gave 3, the gathers 1.5).
+// times as long.  H = 16, 144 chunks / 520 chunks of 15 documents / 36 chunks, in a step's kernel
+// trace: 133 -> 130 / 424 -> 415 / 44.0 -> 42.2 us.
 // Barriers order LDS only (s_waitcnt lgkmcnt(0); s_barrier): global stores stay
 // in flight across them, and the one barrier that needs the dVn tile's copies
 // waits for vector memory explicitly.

@@ -336,9 +336,9 @@ __global__ __launch_bounds__(256, 3) void fwd_prep_kernel(
   }
   // The outputs leave as whole rows through LDS (a store whose lanes are rows takes the
   // vector memory unit 2.5 times as long; with V read by row pieces instead of column
-  // gathers: H = 16, 144 / 520 / 36 / 5 chunks 60.0 -> 51.5 / 198 -> 154 / 21.0 -> 19.1 /
-  // 13.2 -> 11.9 us, 4.1 and 4.9 TB/s on the two long ones): Kg^T from the solve's region, -W through the
-  // K rows' place, then U^T through the solve's region.
+  // gathers: H = 16, 144 / 520 / 36 / 5 chunks 62.6 -> 55.2 / 196 -> 160 / 21.0 -> 19.2 /
+  // 13.4 -> 12.3 us in a step's kernel trace, 3.8 and 4.7 TB/s on the two long ones): Kg^T from the
+  // solve's region, -W through the K rows' place, then U^T through the solve's region.
   __syncthreads();  // the KgT tile is complete, every read of beta gam K is done
   {
     E* kgt = KgT + cb * (D * CH);
@@ -413,14 +413,16 @@ __global__ __launch_bounds__(256, 3) void fwd_prep_kernel(
 // Operands are requested SCAN_DEPTH steps ahead into registers (and four LDS rings);
 // 3, 5 or 6 steps measured the same.  Half of a step's requests go out in each of its
 // two waits (Kg^T a step later than -W): all at once they filled the memory unit's queue
-// and held up the wave's MFMAs (H = 16 / 4, 144 chunks: 84.5 -> 80.7 / 74.6 -> 72.8 us,
-// the reverse scan 93.4 -> 92 / 83.5 -> 77.9; 36 chunks 23.1 -> 22.0, 25.3 -> 24.2).  No step computes an address (ScanBlocks, ScanTable)
+// and held up the wave's MFMAs (each scan alone, H = 16 / 4, 144 chunks: 84.5 -> 80.7 /
+// 74.6 -> 72.8 us, the reverse scan 93.4 -> 92 / 83.5 -> 77.9; 36 chunks 23.1 -> 22.0,
+// 25.3 -> 24.2).  No step computes an address (ScanBlocks, ScanTable)
 // and nothing in a round is conditional, so the compiler's own waits leave every later
 // request in flight; the first round is peeled because a loop entered with fewer
 // operations in flight than it runs with waits as strictly as its entry.
 //
-// Measured (H = 16, one document of 144 chunks / 15 documents, 520 chunks): 102.6 -> 80.7
-// us, 294 -> 240 us; 36 chunks 29.1 -> 22.0; four heads, 144 chunks 97.9 -> 72.8.  LDS
+// Measured in the kernel trace of whole steps (H = 16, one document of 144 chunks / 15
+// documents, 520 chunks): 107 -> 85 us, 298 -> 249 us; 36 chunks 29.7 -> 22.0; four heads,
+// 144 chunks 98.6 -> 73.3.  LDS
 // went from 136 KB to 72 KB a workgroup, so two share a CU.
 //
 // The waits for -W: loads, copies and stores of a wave retire in issue order, so a copy
@@ -610,9 +612,9 @@ __global__ __launch_bounds__(SCAN_THREADS, 2) void fwd_scan_kernel(
 // ---------------------------------------------------------------------------
 // fwd_out: O^T (v rows, t columns) per chunk and head.  h^T and v_new^T come in by row
 // pieces (operand_from_rows) and O leaves as whole rows: H = 16, 144 / 520 / 36 / 5 chunks
-// 46.6 -> 43.6 / 152.7 -> 146.8 / 16.5 -> 15.9 / 7.9 -> 7.2 us against fragments read and
-// O stored with lanes on 16 different rows.  Bound by HBM on the long ones: 222 MB at 5.1
-// TB/s (a large copy reaches 5.2).
+// 44.3 -> 41.7 / 152 -> 144 / 16.2 -> 15.2 / 7.1 -> 7.2 us in a step's kernel trace, against
+// fragments read and O stored with lanes on 16 different rows.  Bound by HBM on the long ones:
+// 228 MB at 5.5 TB/s, some of it from the memory-side cache (a large copy reaches 5.2).
 // ---------------------------------------------------------------------------
 template <class I, class E>  // I: element type of q, k and o; E: operand type (as fwd_prep)
 __global__ __launch_bounds__(256) void fwd_out_kernel(
